@@ -116,6 +116,8 @@ struct DeviceState {
   void *stage[kStageBufs] = {};
   hipEvent_t stage_ev[kStageBufs] = {};
   bool stage_pending[kStageBufs] = {};
+  // words of pinned host memory that kernels write results to (host_words)
+  uint32_t *host_words = nullptr;
   // measurement
   std::vector<hipEvent_t> events;
   std::vector<hipEvent_t> kevents;  // per-kernel timers
@@ -445,6 +447,20 @@ int status_collect(DeviceState &ds, hipStream_t s) {
     g_last_error = "input holds a centroid id or code out of range";
     return TAC_ERR_INVALID_ARGUMENT;
   }
+  return TAC_OK;
+}
+
+// Pinned host words that a call's kernels write their flags and small results
+// to: read once the stream is synchronised, with no copy in between (a copy
+// of one word takes a 4 us kernel of its own and its launch).  A call sets
+// the words it uses before its launch and holds the device's lock until it
+// has read them.
+constexpr uint32_t kHostWords = 16;
+int host_words(DeviceState &ds) {
+  if (ds.host_words) return TAC_OK;
+  void *p = nullptr;
+  HIP_TRY(hipHostMalloc(&p, kHostWords * sizeof(uint32_t), hipHostMallocDefault));
+  ds.host_words = static_cast<uint32_t *>(p);
   return TAC_OK;
 }
 
@@ -1791,6 +1807,8 @@ int tac_gpu_release_workspace(void) {
     b->ptr = nullptr;
     b->bytes = 0;
   }
+  if (ds->host_words) HIP_TRY(hipHostFree(ds->host_words));
+  ds->host_words = nullptr;
   for (int b = 0; b < DeviceState::kStageBufs; ++b) {
     if (ds->stage[b]) HIP_TRY(hipHostFree(ds->stage[b]));
     if (ds->stage_ev[b]) HIP_TRY(hipEventDestroy(ds->stage_ev[b]));
@@ -2373,12 +2391,15 @@ int crc_core(DeviceState &ds, hipStream_t s, const uint8_t *d_buf, uint64_t len,
   return TAC_OK;
 }
 
-int refine_smem(uint32_t n_q, uint32_t dim, size_t *bytes) {
+// The shapes refine takes: the query tokens and four waves' centroid rows (a
+// row per slot, in 640 floats) and best values within 64 KB, as the header
+// states.  refine_kernel's own LDS stays below kCandLdsMax for all of them.
+int refine_fits(uint32_t n_q, uint32_t dim) {
   if (dim > 4096 || n_q > 65536) return TAC_ERR_UNSUPPORTED;
-  const uint64_t floats = refine_lds_floats(n_q, dim);
-  if (floats * sizeof(float) > 65536) return TAC_ERR_UNSUPPORTED;
-  *bytes = (size_t)floats * sizeof(float);
-  return TAC_OK;
+  uint32_t s = 64 / refine_qp(n_q);
+  while (s > 1 && s * (dim + 1) > 640) s >>= 1;
+  const uint64_t floats = (uint64_t)n_q * (dim + 1) + 4 * (s * (dim + 1) + 128);
+  return floats * sizeof(float) > 65536 ? TAC_ERR_UNSUPPORTED : TAC_OK;
 }
 
 // refine.zig:99-105 argument checks, shared by both entry points.
@@ -2388,37 +2409,64 @@ int validate_refine(const tac_doc_index *ix, uint64_t table_len, uint32_t n_q) {
   if (table_len != (uint64_t)ix->m * ix->ksub * n_q) return TAC_ERR_TABLE_SIZE_MISMATCH;
   if (ix->dim == 0 || ix->m == 0 || ix->ksub == 0 || ix->ksub > 65536)
     return TAC_ERR_INVALID_ARGUMENT;
-  size_t smem;
-  return refine_smem(n_q, ix->dim, &smem);
+  return refine_fits(n_q, ix->dim);
+}
+
+// Up to 512 candidates, or rows past 64 floats: 8 waves a block and tiles of
+// 128 tokens, so that a document is one or two steps long; more candidates
+// fill the chip by themselves and take 4 waves and tiles of 64, whose LDS
+// lets 5 blocks share a CU.  Call times in us (8 waves x 128 | 4 x 64; 32
+// query tokens, m16, documents of 1-100 tokens): dim 64 at 250 candidates
+// 36.2 | 42.7, 500 39.0 | 44.6, 1,000 53.6 | 48.9, 4,000 130 | 106; dim 128
+// at 1,000 67.9 | 78.3, 4,000 169 | 207.
+template <int R, bool FAST>
+int refine_launch(const RefineIndex &r, const float *d_q, uint32_t n_q, const float *d_table,
+                  const uint32_t *d_ids, uint32_t n_cand, float *d_scores,
+                  unsigned long long *first_bad, uint32_t *any_bad, hipStream_t s) {
+  const bool wide = n_cand <= 512 || r.dim > 64;
+  const uint32_t waves = wide ? 8 : 4, tile = refine_tile(r.dim, r.M, wide ? 128 : 64);
+  const uint32_t lds =
+      (uint32_t)(refine_lds_floats(n_q, r.dim, FAST, waves, r.M, tile) * sizeof(float));
+  if (int st = raise_lds((const void *)refine_kernel<R, FAST>, lds, 0)) return st;
+  const unsigned blocks = n_cand < 16384 ? n_cand : 16384;
+  refine_kernel<R, FAST><<<blocks, 64 * waves, lds, s>>>(r, d_q, n_q, d_table, d_ids, n_cand,
+                                                         tile, d_scores, first_bad, any_bad);
+  LAUNCH_TRY("refine_kernel");
+  return TAC_OK;
 }
 
 int refine_core(DeviceState &ds, hipStream_t s, const tac_doc_index &ix, const float *d_table,
                 const float *d_q, uint32_t n_q, const uint32_t *d_ids, uint32_t n_cand,
                 float *d_scores) {
-  size_t smem = 0;
-  int st = refine_smem(n_q, ix.dim, &smem);
-  if (st) return st;
-  if ((st = ensure(ds, ds.io_x3, (size_t)n_cand * sizeof(uint32_t) + 16))) return st;
-  uint32_t *status = as<uint32_t>(ds.io_x3);
-  uint32_t *first_bad = status + n_cand;
-  HIP_TRY(hipMemsetAsync(first_bad, 0xFF, sizeof(uint32_t), s));
+  // The failing candidate's word stays all ones between calls: only a call
+  // that raised the host flag has to read it back and restore it.
+  int st;
+  if ((st = host_words(ds))) return st;
+  if (!ds.io_x3.ptr) {
+    if ((st = ensure(ds, ds.io_x3, sizeof(unsigned long long)))) return st;
+    HIP_TRY(hipMemsetAsync(ds.io_x3.ptr, 0xFF, sizeof(unsigned long long), s));
+  }
+  unsigned long long *first_bad = as<unsigned long long>(ds.io_x3);
+  uint32_t *any_bad = ds.host_words;
+  *any_bad = 0;
   RefineIndex r{ix.centroids, ix.doc_index, ix.doc_payload, ix.doc_token_offsets,
                 ix.residual_norms, ix.n_docs, ix.n_tokens, ix.payload_len, ix.dim, ix.kappa,
                 ix.m, ix.ksub};
-  const uint32_t want = (n_cand + kRefineWaves - 1) / kRefineWaves;
-  const unsigned blocks = want < 8192 ? want : 8192;
   const bool profile = g_profile;
   hipEvent_t ea = nullptr, eb = nullptr;
   if (profile) {
     if ((st = event_at(ds, 0, &ea)) || (st = event_at(ds, 1, &eb))) return st;
     HIP_TRY(hipEventRecord(ea, s));
   }
-  refine_kernel<<<blocks, 64 * kRefineWaves, smem, s>>>(r, d_q, n_q, d_table, d_ids, n_cand,
-                                                       d_scores, status, first_bad);
-  LAUNCH_TRY("refine_kernel");
+  const bool fast = (ix.dim == 64 || ix.dim == 128) && (uintptr_t)ix.centroids % 16 == 0 &&
+                    (uintptr_t)d_q % 16 == 0;
+  // Two tokens a lane when a wave covers at most two (n_q > 16), else one.
+  const bool two = fast && n_q > 16;
+  auto *launch = two ? refine_launch<2, true> : fast ? refine_launch<1, true>
+                                                     : refine_launch<1, false>;
+  st = launch(r, d_q, n_q, d_table, d_ids, n_cand, d_scores, first_bad, any_bad, s);
+  if (st) return st;
   if (profile) HIP_TRY(hipEventRecord(eb, s));
-  uint32_t bad = 0xFFFFFFFFu;
-  HIP_TRY(hipMemcpyAsync(&bad, first_bad, sizeof(bad), hipMemcpyDeviceToHost, s));
   HIP_TRY(hipStreamSynchronize(s));
   if (profile) {
     float ms = 0.0f;
@@ -2427,11 +2475,13 @@ int refine_core(DeviceState &ds, hipStream_t s, const tac_doc_index &ix, const f
     g_prof.refine_ms += ms;
     g_prof.refine_launches += 1;
   }
-  if (bad != 0xFFFFFFFFu) {
-    uint32_t code = 0;
-    HIP_TRY(hipMemcpy(&code, status + bad, sizeof(code), hipMemcpyDeviceToHost));
-    g_last_error = "refine failed at candidate " + std::to_string(bad);
-    return (int)code;
+  if (__atomic_load_n(any_bad, __ATOMIC_ACQUIRE)) {
+    unsigned long long bad = 0;
+    HIP_TRY(hipMemcpyAsync(&bad, first_bad, sizeof(bad), hipMemcpyDeviceToHost, s));
+    HIP_TRY(hipMemsetAsync(first_bad, 0xFF, sizeof(bad), s));
+    HIP_TRY(hipStreamSynchronize(s));
+    g_last_error = "refine failed at candidate " + std::to_string(bad >> 32);
+    return (int)(bad & 0xFFFFFFFFu);
   }
   return TAC_OK;
 }
