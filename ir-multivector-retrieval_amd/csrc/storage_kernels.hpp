@@ -269,27 +269,38 @@ __global__ __launch_bounds__(256) void doc_write_kernel(
 // CRC-32/ISO-HDLC of a device buffer (std.hash.Crc32, as storage.zig applies
 // it to the whole image before the footer, :612-617, :782-786).
 //
-// Reflected representation: bit 31 holds the coefficient of x^0.  The
-// register after bytes B starting from register r is
-//   crc(r, B) = crc(0, B) ^ (r * x^(8|B|) mod P),
-// so zero-seeded CRCs of consecutive pieces combine left to right by one
-// modular multiplication each.  The buffer splits into an unaligned head
-// (< 16 bytes), a body of whole kCrcLeaf-byte leaves and a tail
-// (< kCrcLeaf bytes).  A thread owns one leaf and runs kCrcWays interleaved
-// slicing-by-8 chains over its consecutive sub-leaves (independent LDS
-// lookups in flight), joins them, the 256 leaves of a block combine in an
-// LDS tree, one block combines the block results, and one thread adds head,
-// tail and the all-ones preset.
+// Polynomials over GF(2) mod P, reflected: bit 31 holds the coefficient of
+// x^0, so a little-endian word of the buffer is a polynomial as it stands.
+// The CRC of n bytes B is B(x) x^32 + ones(x) x^(8n) mod P, complemented.
+// The kernel evaluates B(x), padded with zero bytes to whole blocks, and the
+// host applies x^32, the inverse of the padding and the preset.
+//
+// A block owns consecutive chunks of kCrcChunk bytes and walks them in steps
+// of 8 KB: every lane loads 16 bytes a step (coalesced, a chunk's loads in
+// flight at once) into four Horner sums of one word each, s <- s x^(8 * 8192)
+// + word.  The product by a constant is four LDS table reads, one a byte of
+// s.  What is left is the 8 KB polynomial of the block's 512 lanes: each lane
+// joins its four words and multiplies by its own power of x, the block XORs
+// the lanes and multiplies by x^(8 * bytes behind its chunks), and stores one
+// word to pinned host memory, where the host XORs the blocks' words.
+//
+// Bound by the table reads in LDS (one a byte and lane, random banks) and by
+// latency.  One leaf of 256 bytes a thread read the buffer 64 lines an
+// instruction and built its tables in every block, and one more block joined
+// the results in a chain: 20 + 25 us for 30.6 MB.  This kernel takes 14 us; with the lanes
+// and waves folded in a tree by one wave and the blocks XORed by device
+// atomics on one word it took 24.
 // ---------------------------------------------------------------------------
 constexpr uint32_t kCrcPoly = 0xEDB88320u;
-constexpr uint32_t kCrcLeaf = 256;       // bytes per thread (power of two)
-constexpr uint32_t kCrcLeafLog2 = 8;
-constexpr uint32_t kCrcWays = 4;         // interleaved chains per thread
-constexpr uint32_t kCrcSub = kCrcLeaf / kCrcWays;  // 64 bytes per chain
-constexpr uint32_t kCrcSubLog2 = 6;
-constexpr int kCrcBlock = 256;
+constexpr uint32_t kCrcInvX = 0xDB710641u;  // x^-1 mod P
+constexpr uint32_t kCrcOne = 0x80000000u;   // x^0
+constexpr uint32_t kCrcThreads = 512;
+constexpr uint32_t kCrcSteps = 8;  // loads of a lane in flight
+constexpr uint32_t kCrcStepBytes = kCrcThreads * 16;
+constexpr uint32_t kCrcChunk = kCrcSteps * kCrcStepBytes;
+constexpr uint32_t kCrcBlocks = 1024;  // most blocks, a host word each
 
-__host__ __device__ inline uint32_t crc_mulmod(uint32_t a, uint32_t b) {
+inline uint32_t crc_mulmod(uint32_t a, uint32_t b) {
   uint32_t p = 0;
   for (int i = 0; i < 32; ++i) {
     if ((a >> (31 - i)) & 1u) p ^= b;
@@ -298,184 +309,141 @@ __host__ __device__ inline uint32_t crc_mulmod(uint32_t a, uint32_t b) {
   return p;
 }
 
-// Multiplication tables for the shifts: tx[j][i] = x^(8 * 2^j) * x^i mod P
-// (j = 0..63, i = 0..31), so r * x^(8 * 2^j) is the XOR of tx[j][i] over the
-// coefficients i that r holds: 32 independent selects instead of a 32-step
-// serial chain.
-constexpr uint32_t kCrcTxRows = 64;
-
-inline void crc_tx_host(uint32_t* tx) {  // [kCrcTxRows][32]
-  uint32_t t = 0x40000000u;  // x^1
-  for (int j = 0; j < 3; ++j) t = crc_mulmod(t, t);  // x^8
-  for (uint32_t j = 0; j < kCrcTxRows; ++j) {
-    uint32_t v = t;  // x^(8 * 2^j) * x^0
-    for (int i = 0; i < 32; ++i) {
-      tx[j * 32 + i] = v;
-      v = (v & 1u) ? (v >> 1) ^ kCrcPoly : v >> 1;  // times x
-    }
-    t = crc_mulmod(t, t);
-  }
-}
-
-// Branch-free: every row entry is loaded (eight 16-byte LDS reads) and
-// masked by its coefficient bit.
-__device__ __forceinline__ uint32_t crc_mul_row(uint32_t r, const uint32_t* row) {
-  const uint4* row4 = reinterpret_cast<const uint4*>(row);
-  uint32_t p0 = 0, p1 = 0;
-#pragma unroll
-  for (int q = 0; q < 8; ++q) {
-    const uint4 v = row4[q];
-    const int i = 4 * q;
-    p0 ^= v.x & (0u - ((r >> (31 - i)) & 1u));
-    p1 ^= v.y & (0u - ((r >> (30 - i)) & 1u));
-    p0 ^= v.z & (0u - ((r >> (29 - i)) & 1u));
-    p1 ^= v.w & (0u - ((r >> (28 - i)) & 1u));
-  }
-  return p0 ^ p1;
-}
-
-// r * x^(8 * count * 2^shift) mod P with tx rows in LDS (one row per set bit).
-__device__ __forceinline__ uint32_t crc_shift_tx(uint32_t r, uint64_t count, uint32_t shift,
-                                                 const uint32_t* tx) {
-  while (count) {
-    const uint32_t j = (uint32_t)__builtin_ctzll(count);
-    r = crc_mul_row(r, tx + (j + shift) * 32);
-    count &= count - 1;
-  }
+// base^e mod P.
+inline uint32_t crc_pow(uint32_t base, uint64_t e) {
+  uint32_t r = kCrcOne;
+  for (; e; e >>= 1, base = crc_mulmod(base, base))
+    if (e & 1u) r = crc_mulmod(r, base);
   return r;
 }
 
-// Slicing-by-8 tables in LDS: T[k][i] = CRC contribution of byte value i
-// followed by k zero bytes, from a zero register.
-__device__ inline void crc_tables(uint32_t (*T)[256]) {
-  for (uint32_t i = threadIdx.x; i < 256; i += blockDim.x) {
-    uint32_t r = i;
-    for (int k = 0; k < 8; ++k) r = (r & 1u) ? (r >> 1) ^ kCrcPoly : r >> 1;
-    T[0][i] = r;
+// Device tables, in words: products of the four bytes of a word by x^(8 *
+// kCrcStepBytes) and by x^32, entry [byte][value]; x^(128 i), the weight of
+// the lane i places before the last; and the powers x^(8 kCrcChunk i 256^l),
+// entry [l][i].
+constexpr uint32_t kCrcTabStep = 0, kCrcTabWord = 1024, kCrcTabLane = 2048,
+                   kCrcTabPow = kCrcTabLane + kCrcThreads, kCrcTabWords = kCrcTabPow + 1024;
+
+inline void crc_tables_host(uint32_t* t) {
+  const uint32_t x = kCrcOne >> 1;
+  const uint32_t by[2] = {crc_pow(x, 8ull * kCrcStepBytes), crc_pow(x, 32)};
+  for (uint32_t k = 0; k < 2; ++k)
+    for (uint32_t b = 0; b < 4; ++b)
+      for (uint32_t v = 0; v < 256; ++v)
+        t[k * 1024 + b * 256 + v] = crc_mulmod(v << (8 * b), by[k]);
+  uint32_t unit = crc_pow(x, 128), p = kCrcOne;
+  for (uint32_t i = 0; i < kCrcThreads; ++i, p = crc_mulmod(p, unit)) t[kCrcTabLane + i] = p;
+  unit = crc_pow(x, 8ull * kCrcChunk);
+  for (uint32_t l = 0; l < 4; ++l) {
+    p = kCrcOne;
+    for (uint32_t i = 0; i < 256; ++i, p = crc_mulmod(p, unit)) t[kCrcTabPow + l * 256 + i] = p;
+    unit = p;  // unit^256
   }
-  __syncthreads();
-  for (int k = 1; k < 8; ++k) {
-    for (uint32_t i = threadIdx.x; i < 256; i += blockDim.x) {
-      const uint32_t v = T[k - 1][i];
-      T[k][i] = (v >> 8) ^ T[0][v & 0xFFu];
+}
+
+// The CRC of len bytes from the kernel's polynomial over the bytes and `pad`
+// zero bytes behind them.
+inline uint32_t crc_finish(uint32_t raw, uint32_t x32_over_pad, uint32_t preset) {
+  return crc_mulmod(raw, x32_over_pad) ^ preset ^ 0xFFFFFFFFu;
+}
+
+// s times the table's constant.
+__device__ __forceinline__ uint32_t crc_times(uint32_t s, const uint32_t* tab) {
+  return tab[s & 0xFFu] ^ tab[256 + ((s >> 8) & 0xFFu)] ^ tab[512 + ((s >> 16) & 0xFFu)] ^
+         tab[768 + (s >> 24)];
+}
+
+// a b mod P: the 64-bit carry-less product, its low word (the powers from
+// x^32 on) reduced through the x^32 table.
+__device__ __forceinline__ uint32_t crc_mul(uint32_t a, uint32_t b, const uint32_t* word_tab) {
+  uint32_t lo = 0, hi = 0;  // of the product shifted left by one
+#pragma unroll
+  for (int i = 0; i < 32; ++i) {
+    const uint32_t m = (uint32_t)((int32_t)(a << (31 - i)) >> 31);
+    if (i < 31) lo ^= (b << (i + 1)) & m;
+    hi ^= (b >> (31 - i)) & m;
+  }
+  return hi ^ crc_times(lo, word_tab);
+}
+
+// The 16 bytes at `pos` from base (16-byte aligned); bytes outside
+// [first, end) are zero and not read.
+__device__ __forceinline__ uint4 crc_load(const uint8_t* base, uint64_t pos, uint64_t first,
+                                          uint64_t end) {
+  if (pos >= first && pos + 16 <= end) return *reinterpret_cast<const uint4*>(base + pos);
+  uint32_t v[4] = {0, 0, 0, 0};
+  if (pos + 16 > first && pos < end)
+    for (uint32_t b = 0; b < 16; ++b)
+      if (pos + b >= first && pos + b < end) v[b / 4] |= (uint32_t)base[pos + b] << (8 * (b % 4));
+  return make_uint4(v[0], v[1], v[2], v[3]);
+}
+
+// Bytes [first, end) from base, n_chunks chunks, `per` to a block; block b's
+// word goes to host_out[b].
+__global__ __launch_bounds__(kCrcThreads) void crc_kernel(
+    const uint8_t* __restrict__ base, uint64_t first, uint64_t end, uint32_t n_chunks,
+    uint32_t per, const uint32_t* __restrict__ tables, uint32_t* __restrict__ host_out) {
+  __shared__ __attribute__((aligned(16))) uint32_t tab[2 * 1024];
+  __shared__ uint32_t wave_word[kCrcThreads / 64];
+  __shared__ uint32_t weight;
+  const uint32_t t = threadIdx.x;
+  const uint32_t c0 = blockIdx.x * per;
+  const uint32_t c1 = n_chunks - c0 < per ? n_chunks : c0 + per;
+  uint4 v[kCrcSteps];
+  auto load = [&](uint32_t c) {
+    const uint64_t lo = (uint64_t)c * kCrcChunk;
+    if (lo >= first && lo + kCrcChunk <= end) {
+      const uint4* p = reinterpret_cast<const uint4*>(base + lo) + t;
+#pragma unroll
+      for (uint32_t j = 0; j < kCrcSteps; ++j) v[j] = p[j * kCrcThreads];
+    } else {
+#pragma unroll
+      for (uint32_t j = 0; j < kCrcSteps; ++j)
+        v[j] = crc_load(base, lo + j * kCrcStepBytes + t * 16, first, end);
     }
-    __syncthreads();
-  }
-}
-
-// Eight bytes (lo = bytes 0-3, hi = bytes 4-7, little-endian): byte j needs
-// the table with 7 - j trailing zero bytes.
-__device__ __forceinline__ uint32_t crc_step8(uint32_t r, uint32_t lo, uint32_t hi,
-                                              const uint32_t (*T)[256]) {
-  r ^= lo;
-  return T[7][r & 0xFFu] ^ T[6][(r >> 8) & 0xFFu] ^ T[5][(r >> 16) & 0xFFu] ^ T[4][r >> 24] ^
-         T[3][hi & 0xFFu] ^ T[2][(hi >> 8) & 0xFFu] ^ T[1][(hi >> 16) & 0xFFu] ^ T[0][hi >> 24];
-}
-
-struct CrcNode {
-  uint32_t crc;
-  uint32_t leaves;
-};
-
-__device__ __forceinline__ CrcNode crc_join(CrcNode a, CrcNode b, const uint32_t* tx) {
-  if (!b.leaves) return a;
-  return CrcNode{crc_shift_tx(a.crc, b.leaves, kCrcLeafLog2, tx) ^ b.crc, a.leaves + b.leaves};
-}
-
-// Combines the block's 256 nodes in order (one per thread, `mine`): a
-// shuffle tree inside each wave, then one thread joins the four wave results.
-// Every thread returns the block's combination.
-__device__ inline CrcNode crc_block_combine(CrcNode mine, CrcNode* wave_res, const uint32_t* tx) {
-  const uint32_t lane = threadIdx.x % 64, w = threadIdx.x / 64;
-  for (uint32_t span = 1; span < 64; span <<= 1) {
-    const CrcNode other{__shfl_down(mine.crc, span, 64), __shfl_down(mine.leaves, span, 64)};
-    if (lane % (2 * span) == 0 && lane + span < 64) mine = crc_join(mine, other, tx);
-  }
-  if (lane == 0) wave_res[w] = mine;
+  };
+  load(c0);
+  for (uint32_t f = t; f < 2 * 1024 / 4; f += kCrcThreads)
+    reinterpret_cast<uint4*>(tab)[f] = reinterpret_cast<const uint4*>(tables)[f];
+  const uint32_t lane_weight = tables[kCrcTabLane + kCrcThreads - 1 - t];
+  // the chunks behind the block, in base 256: the last wave's first lane
+  // multiplies their powers while the others fold
+  const uint32_t behind = n_chunks - c1;
+  uint32_t pw[4];
+#pragma unroll
+  for (uint32_t l = 0; l < 4; ++l)
+    pw[l] = tables[kCrcTabPow + l * 256 + ((behind >> (8 * l)) & 0xFFu)];
   __syncthreads();
-  if (threadIdx.x == 0) {
-    CrcNode acc = wave_res[0];
-    for (uint32_t q = 1; q < kCrcBlock / 64; ++q) acc = crc_join(acc, wave_res[q], tx);
-    wave_res[0] = acc;
-  }
-  __syncthreads();
-  const CrcNode out = wave_res[0];
-  __syncthreads();
-  return out;
-}
-
-// Leaves of the 16-byte aligned body: every block reduces its 256 leaves to
-// one CrcNode.  g_tx is the [64][32] shift table in global memory.
-__global__ __launch_bounds__(kCrcBlock) void crc_leaf_kernel(const uint8_t* __restrict__ body,
-                                                             uint64_t n_leaves,
-                                                             const uint32_t* __restrict__ g_tx,
-                                                             CrcNode* __restrict__ nodes) {
-  __shared__ uint32_t T[8][256];
-  __shared__ __attribute__((aligned(16))) uint32_t tx[kCrcTxRows * 32];
-  __shared__ CrcNode node[kCrcBlock / 64];
-  for (uint32_t f = threadIdx.x; f < kCrcTxRows * 32; f += kCrcBlock) tx[f] = g_tx[f];
-  crc_tables(T);  // synchronises
-  const uint64_t leaf = (uint64_t)blockIdx.x * kCrcBlock + threadIdx.x;
-  uint32_t r = 0;
-  uint32_t have = 0;
-  if (leaf < n_leaves) {
-    const uint4* p = reinterpret_cast<const uint4*>(body + leaf * kCrcLeaf);
-    uint4 v[kCrcWays][kCrcSub / 16];
+  uint32_t s[4] = {0, 0, 0, 0};
+  for (uint32_t c = c0;;) {
 #pragma unroll
-    for (uint32_t w = 0; w < kCrcWays; ++w)
+    for (uint32_t j = 0; j < kCrcSteps; ++j) {
+      const uint32_t word[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
 #pragma unroll
-      for (uint32_t q = 0; q < kCrcSub / 16; ++q) v[w][q] = p[w * (kCrcSub / 16) + q];
-    uint32_t rw[kCrcWays];
-#pragma unroll
-    for (uint32_t w = 0; w < kCrcWays; ++w) rw[w] = 0;
-#pragma unroll
-    for (uint32_t q = 0; q < kCrcSub / 16; ++q)
-#pragma unroll
-      for (uint32_t w = 0; w < kCrcWays; ++w) {
-        rw[w] = crc_step8(rw[w], v[w][q].x, v[w][q].y, T);
-        rw[w] = crc_step8(rw[w], v[w][q].z, v[w][q].w, T);
-      }
-    r = rw[0];
-#pragma unroll
-    for (uint32_t w = 1; w < kCrcWays; ++w) r = crc_mul_row(r, tx + kCrcSubLog2 * 32) ^ rw[w];
-    have = 1;
-  }
-  const CrcNode blk = crc_block_combine(CrcNode{r, have}, node, tx);
-  if (threadIdx.x == 0) nodes[blockIdx.x] = blk;
-}
-
-// One block: folds the block nodes in order, then head, body and tail.
-__global__ __launch_bounds__(kCrcBlock) void crc_final_kernel(
-    const uint8_t* __restrict__ buf, uint64_t head, uint64_t n_leaves, uint64_t tail,
-    const CrcNode* __restrict__ nodes, uint32_t n_nodes, const uint32_t* __restrict__ g_tx,
-    uint32_t* __restrict__ crc_out) {
-  __shared__ uint32_t T[8][256];
-  __shared__ __attribute__((aligned(16))) uint32_t tx[kCrcTxRows * 32];
-  __shared__ CrcNode node[kCrcBlock / 64];
-  for (uint32_t f = threadIdx.x; f < kCrcTxRows * 32; f += kCrcBlock) tx[f] = g_tx[f];
-  crc_tables(T);  // synchronises
-  CrcNode acc{0, 0};
-  for (uint32_t b0 = 0; b0 < n_nodes; b0 += kCrcBlock) {
-    const uint32_t b = b0 + threadIdx.x;
-    const CrcNode part = crc_block_combine(b < n_nodes ? nodes[b] : CrcNode{0, 0}, node, tx);
-    acc = crc_join(acc, part, tx);
-  }
-  if (threadIdx.x != 0) return;
-  uint32_t rr = 0xFFFFFFFFu;
-  for (uint64_t i = 0; i < head; ++i) rr = T[0][(rr ^ buf[i]) & 0xFFu] ^ (rr >> 8);
-  rr = crc_shift_tx(rr, n_leaves, kCrcLeafLog2, tx) ^ acc.crc;
-  // The tail starts 16-byte aligned (or at byte 0 when the head took all).
-  const uint8_t* t = buf + head + n_leaves * kCrcLeaf;
-  uint64_t i = 0;
-  if (((uintptr_t)t & 7) == 0) {
-    const uint2* t8 = reinterpret_cast<const uint2*>(t);
-    for (; i + 8 <= tail; i += 8) {
-      const uint2 v = t8[i / 8];
-      rr = crc_step8(rr, v.x, v.y, T);
+      for (int q = 0; q < 4; ++q) s[q] = crc_times(s[q], tab + kCrcTabStep) ^ word[q];
     }
+    if (++c >= c1) break;
+    load(c);
   }
-  for (; i < tail; ++i) rr = T[0][(rr ^ t[i]) & 0xFFu] ^ (rr >> 8);
-  *crc_out = rr ^ 0xFFFFFFFFu;
+  uint32_t r = s[0];
+#pragma unroll
+  for (int q = 1; q < 4; ++q) r = crc_times(r, tab + kCrcTabWord) ^ s[q];
+  r = crc_mul(r, lane_weight, tab + kCrcTabWord);
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) r ^= __shfl_xor(r, off, 64);
+  if (t % 64 == 0) wave_word[t / 64] = r;
+  if (t == kCrcThreads - 64) {
+    uint32_t f = pw[0];
+    for (uint32_t l = 1; l < 4 && behind >> (8 * l); ++l)
+      f = crc_mul(f, l == 1 ? pw[1] : l == 2 ? pw[2] : pw[3], tab + kCrcTabWord);
+    weight = f;
+  }
+  __syncthreads();
+  if (t != 0) return;
+#pragma unroll
+  for (uint32_t ww = 1; ww < kCrcThreads / 64; ++ww) r ^= wave_word[ww];
+  __hip_atomic_store(host_out + blockIdx.x, crc_mul(r, weight, tab + kCrcTabWord),
+                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 }  // namespace tacgpu

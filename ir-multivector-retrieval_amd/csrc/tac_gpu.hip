@@ -98,7 +98,7 @@ struct DeviceState {
   // training / encode workspace
   Buffer xs, codes, e, hist, counts, start, sorted, flags, scal, trace, io_in, io_out, io_cb,
       io_init, counter, kpp_state, kpp_w, kpp_bsum, kpp_bad, status, io_aux, io_out2, scan_sums,
-      io_x1, io_x2, io_x3, crc_tx, fold_pre, fold_chunks, cand_nbr, cand_defer, cand_count, cand_anchor, cand_grid, kpp_src,
+      io_x1, io_x2, io_x3, crc_tables, fold_pre, fold_chunks, cand_nbr, cand_defer, cand_count, cand_anchor, cand_grid, kpp_src,
       fold_order, cell_par, cell_cids, cell_ccnt, cell_rec, cell_list;
   // token-aware clustering
   Buffer tac_v, tac_idx, tac_offs, tac_G, tac_spreads, tac_w, tac_e, tac_code, tac_sorted,
@@ -107,7 +107,6 @@ struct DeviceState {
       tac_chl, tac_cprob, tac_inv, tac_rsum, tac_ranges, tac_h, tac_ktiles, tac_big, tac_ids,
       tac_pcnt, tac_pslots;
   hipEvent_t tac_pre_ev[16] = {};  // chunk arrivals for the early spreads (a ring)
-  bool crc_tx_ready = false;
   // training's second stream (two halves of the subspaces) and its events
   hipStream_t aux_stream[1] = {};
   hipEvent_t aux_fork = nullptr, aux_join[1] = {};
@@ -455,7 +454,7 @@ int status_collect(DeviceState &ds, hipStream_t s) {
 // of one word takes a 4 us kernel of its own and its launch).  A call sets
 // the words it uses before its launch and holds the device's lock until it
 // has read them.
-constexpr uint32_t kHostWords = 16;
+constexpr uint32_t kHostWords = kCrcBlocks;
 int host_words(DeviceState &ds) {
   if (ds.host_words) return TAC_OK;
   void *p = nullptr;
@@ -1789,7 +1788,7 @@ int tac_gpu_release_workspace(void) {
                     &ds->io_in,     &ds->io_out,  &ds->io_cb,     &ds->io_init,  &ds->counter,
                     &ds->kpp_state, &ds->kpp_w,   &ds->kpp_bsum,  &ds->kpp_bad,  &ds->status,
                     &ds->io_aux,    &ds->io_out2, &ds->scan_sums, &ds->io_x1,    &ds->io_x2,
-                    &ds->io_x3,     &ds->crc_tx,  &ds->fold_pre,  &ds->fold_chunks,
+                    &ds->io_x3,     &ds->crc_tables, &ds->fold_pre,  &ds->fold_chunks,
                     &ds->tac_v,     &ds->tac_idx, &ds->tac_offs,  &ds->tac_G,
                     &ds->tac_spreads, &ds->tac_w, &ds->tac_e,     &ds->tac_code,
                     &ds->tac_sorted, &ds->tac_tsum, &ds->tac_hist, &ds->tac_counts,
@@ -1801,7 +1800,6 @@ int tac_gpu_release_workspace(void) {
                     &ds->cand_defer, &ds->cand_count, &ds->cand_anchor, &ds->cand_grid,
                     &ds->kpp_src,   &ds->fold_order, &ds->tac_h, &ds->tac_ktiles,
                     &ds->tac_big};
-  ds->crc_tx_ready = false;
   for (Buffer *b : bufs) {
     if (b->ptr) HIP_TRY(hipFree(b->ptr));
     b->ptr = nullptr;
@@ -2346,41 +2344,45 @@ int doc_layouts_core(DeviceState &ds, hipStream_t s, const uint64_t *d_off, uint
 }
 
 int crc_core(DeviceState &ds, hipStream_t s, const uint8_t *d_buf, uint64_t len, uint32_t *out) {
-  const uint64_t mis = (uintptr_t)d_buf % 16;
-  const uint64_t head = mis ? ((16 - mis) < len ? (16 - mis) : len) : 0;
-  const uint64_t leaves = (len - head) / kCrcLeaf;
-  const uint64_t tail = len - head - leaves * kCrcLeaf;
-  const uint64_t nb = (leaves + kCrcBlock - 1) / kCrcBlock;
-  if (nb > 0x7FFFFFFFull) return TAC_ERR_UNSUPPORTED;
+  const uint64_t first = (uintptr_t)d_buf % 16, end = first + len;
+  const uint64_t chunks = (end + kCrcChunk - 1) / kCrcChunk;
+  if (chunks > 0x7FFFFFFFull) return TAC_ERR_UNSUPPORTED;
+  const uint32_t per = (uint32_t)((chunks + kCrcBlocks - 1) / kCrcBlocks);
+  const uint32_t nb = (uint32_t)((chunks + per - 1) / per);
   int st;
-  if ((st = ensure(ds, ds.scan_sums, (size_t)(nb ? nb : 1) * sizeof(CrcNode) + 16))) return st;
-  CrcNode *nodes = as<CrcNode>(ds.scan_sums);
-  uint32_t *d_crc = reinterpret_cast<uint32_t *>(nodes + (nb ? nb : 1));
-  if (!ds.crc_tx_ready) {  // the [64][32] shift table, uploaded once per device
-    static const std::vector<uint32_t> host_tx = [] {
-      std::vector<uint32_t> t(kCrcTxRows * 32);
-      crc_tx_host(t.data());
-      return t;
-    }();
-    if ((st = ensure(ds, ds.crc_tx, host_tx.size() * sizeof(uint32_t)))) return st;
-    HIP_TRY(hipMemcpy(ds.crc_tx.ptr, host_tx.data(), host_tx.size() * sizeof(uint32_t),
-                      hipMemcpyHostToDevice));
-    ds.crc_tx_ready = true;
+  if ((st = host_words(ds))) return st;
+  if (!ds.crc_tables.ptr) {  // uploaded once per device
+    std::vector<uint32_t> t(kCrcTabWords);
+    crc_tables_host(t.data());
+    if ((st = ensure(ds, ds.crc_tables, t.size() * sizeof(uint32_t)))) return st;
+    const hipError_t e = hipMemcpy(ds.crc_tables.ptr, t.data(), t.size() * sizeof(uint32_t),
+                                   hipMemcpyHostToDevice);
+    if (e != hipSuccess) {
+      (void)hipFree(ds.crc_tables.ptr);
+      ds.crc_tables = Buffer{};
+      return hip_status("hipMemcpy(crc tables)", e);
+    }
   }
-  const uint32_t *tx = as<uint32_t>(ds.crc_tx);
+  const uint32_t *tables = as<uint32_t>(ds.crc_tables);
   const bool profile = g_profile;
   hipEvent_t a = nullptr, b = nullptr;
   if (profile) {
     if ((st = event_at(ds, 0, &a)) || (st = event_at(ds, 1, &b))) return st;
     HIP_TRY(hipEventRecord(a, s));
   }
-  if (nb) crc_leaf_kernel<<<(unsigned)nb, kCrcBlock, 0, s>>>(d_buf + head, leaves, tx, nodes);
-  crc_final_kernel<<<1, kCrcBlock, 0, s>>>(d_buf, head, leaves, tail, nodes, (uint32_t)nb, tx,
-                                           d_crc);
-  LAUNCH_TRY("crc kernels");
+  crc_kernel<<<nb, kCrcThreads, 0, s>>>(d_buf - first, first, end, (uint32_t)chunks, per, tables,
+                                        ds.host_words);
+  LAUNCH_TRY("crc_kernel");
   if (profile) HIP_TRY(hipEventRecord(b, s));
-  HIP_TRY(hipMemcpyAsync(out, d_crc, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+  // while it runs: x^32 over the zero bytes that fill the last chunk, and the preset
+  const uint64_t pad = chunks * kCrcChunk - end;
+  const uint32_t x = kCrcOne >> 1;
+  const uint32_t over = crc_mulmod(crc_pow(kCrcInvX, 8 * pad), crc_pow(x, 32));
+  const uint32_t preset = crc_mulmod(0xFFFFFFFFu, crc_pow(x, 8 * len));
   HIP_TRY(hipStreamSynchronize(s));
+  uint32_t raw = 0;
+  for (uint32_t i = 0; i < nb; ++i) raw ^= __atomic_load_n(ds.host_words + i, __ATOMIC_ACQUIRE);
+  *out = crc_finish(raw, over, preset);
   if (profile) {
     float ms = 0.0f;
     HIP_TRY(hipEventElapsedTime(&ms, a, b));
