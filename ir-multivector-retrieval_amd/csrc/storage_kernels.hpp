@@ -148,29 +148,54 @@ __device__ __forceinline__ uint64_t doc_bytes(uint64_t n_d, uint32_t m, uint32_t
 
 constexpr int kScanBlock = 256;
 constexpr int kScanPer = 4;  // elements per thread in the u64 scan
+// Documents past kDocSlice tokens are written in slices of as many, each by a
+// wave of its own: one wave would walk them alone long after the others are
+// done.  Sound offsets make at most n_tokens / 256 slices.
+constexpr uint64_t kDocSlice = 512;
+
+struct DocSlice {
+  uint64_t doc;
+  uint64_t at;     // the document's offset within its scan block
+  uint64_t first;  // the slice's first token
+};
+__host__ __device__ inline uint64_t doc_slices_most(uint64_t n_tokens) {
+  return n_tokens / (kDocSlice / 2);
+}
+
+// State of a layout call on the device.  bad and n_slices are zero between
+// calls: doc_sums_scan_kernel moves them to go and slices.
+struct DocState {
+  unsigned long long n_slices;  // slices listed
+  unsigned long long slices;    // n_slices of this call
+  uint32_t bad;                 // an offset decreases or passes n_tokens
+  uint32_t go;                  // the payload fits and the offsets are sound
+};
 
 // Phase 1: per-block exclusive scan of doc sizes into doc_index, block totals
 // into `sums`.
-// Offsets that decrease or pass n_tokens raise `status` (the writer then
-// does not run) and count as empty documents.
+// Offsets that decrease or pass n_tokens raise st->bad (the writer then
+// does not run) and count as empty documents; long documents' slices are listed.
 __global__ __launch_bounds__(kScanBlock) void doc_sizes_scan_kernel(
     const uint64_t* __restrict__ doc_offsets, uint64_t n_docs, uint64_t n_tokens, uint32_t m,
     uint32_t cb, uint64_t* __restrict__ doc_index, uint64_t* __restrict__ sums,
-    uint32_t* __restrict__ status) {
+    DocState* __restrict__ st, DocSlice* __restrict__ slices) {
   __shared__ uint64_t warp_tot[kScanBlock / 64];
   const uint64_t base = (uint64_t)blockIdx.x * kScanBlock * kScanPer + threadIdx.x * kScanPer;
   uint64_t v[kScanPer];
   uint64_t local = 0;
+  uint32_t is_long = 0;
 #pragma unroll
   for (int q = 0; q < kScanPer; ++q) {
     const uint64_t d = base + q;
     v[q] = 0;
     if (d < n_docs) {
       const uint64_t a = doc_offsets[d], b = doc_offsets[d + 1];
-      if (b < a || b > n_tokens)
-        atomicOr(status, 1u);
-      else
+      if (b < a || b > n_tokens) {
+        atomicOr(&st->bad, 1u);
+      } else {
         v[q] = doc_bytes(b - a, m, cb);
+        is_long |= b - a > kDocSlice ? 1u << q : 0u;
+      }
     }
     local += v[q];
   }
@@ -189,15 +214,24 @@ __global__ __launch_bounds__(kScanBlock) void doc_sizes_scan_kernel(
   for (int q = 0; q < kScanPer; ++q) {
     const uint64_t d = base + q;
     if (d < n_docs) doc_index[d] = run;
+    if (is_long >> q & 1u) {
+      const uint64_t n_d = doc_offsets[d + 1] - doc_offsets[d];
+      const uint64_t count = (n_d + kDocSlice - 1) / kDocSlice;
+      const uint64_t at = atomicAdd(&st->n_slices, (unsigned long long)count);
+      for (uint64_t i = 0; i < count && at + i < doc_slices_most(n_tokens); ++i)
+        slices[at + i] = DocSlice{d, run, i * kDocSlice};
+    }
     run += v[q];
   }
   if (threadIdx.x == kScanBlock - 1) sums[blockIdx.x] = before + incl;
 }
 
 // Phase 2 (one block): exclusive scan of the block totals in place; the
-// grand total lands in doc_index[n_docs].
+// grand total lands in doc_index[n_docs].  Decides whether the writer runs and
+// tells the host (host[0] bad offsets, host[1..2] the total).
 __global__ __launch_bounds__(kScanBlock) void doc_sums_scan_kernel(
-    uint64_t* __restrict__ sums, uint32_t nb, uint64_t* __restrict__ doc_index, uint64_t n_docs) {
+    uint64_t* __restrict__ sums, uint32_t nb, uint64_t* __restrict__ doc_index, uint64_t n_docs,
+    uint64_t payload_len, DocState* __restrict__ st, uint32_t* __restrict__ host) {
   __shared__ uint64_t warp_tot[kScanBlock / 64];
   __shared__ uint64_t carry;
   if (threadIdx.x == 0) carry = 0;
@@ -220,48 +254,70 @@ __global__ __launch_bounds__(kScanBlock) void doc_sums_scan_kernel(
     if (threadIdx.x == kScanBlock - 1) carry = before + incl;
     __syncthreads();
   }
-  if (threadIdx.x == 0) doc_index[n_docs] = carry;
+  if (threadIdx.x == 0) {
+    doc_index[n_docs] = carry;
+    st->go = !st->bad && carry <= payload_len;
+    st->slices = st->n_slices;
+    __hip_atomic_store(host, st->bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(host + 1, (uint32_t)carry, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(host + 2, (uint32_t)(carry >> 32), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
+    st->bad = 0;
+    st->n_slices = 0;
+  }
 }
 
-// Phase 3: add each block's carry-in.
-__global__ __launch_bounds__(kScanBlock) void doc_scan_add_kernel(
-    uint64_t* __restrict__ doc_index, const uint64_t* __restrict__ sums, uint64_t n_docs) {
-  const uint64_t base = (uint64_t)blockIdx.x * kScanBlock * kScanPer + threadIdx.x * kScanPer;
-  const uint64_t add = sums[blockIdx.x];
-#pragma unroll
-  for (int q = 0; q < kScanPer; ++q)
-    if (base + q < n_docs) doc_index[base + q] += add;
+// Tokens [k0, k1) of a document of n_d tokens at p, by one wave: n_d (with the
+// first token), the centroid ids, the codes (as 32-bit words when source and
+// size allow; the id array is 4-aligned, as document starts are 8-aligned)
+// and, behind the last token, zero padding.
+__device__ __forceinline__ void doc_copy(uint32_t lane, uint64_t lo, uint64_t n_d, uint64_t k0,
+                                         uint64_t k1, uint8_t* p, const uint32_t* assign,
+                                         const uint8_t* codes, uint32_t m, uint32_t cb) {
+  uint32_t* ids = reinterpret_cast<uint32_t*>(p + 4);
+  if (lane == 0 && k0 == 0) *reinterpret_cast<uint32_t*>(p) = (uint32_t)n_d;
+  for (uint64_t k = k0 + lane; k < k1; k += 64) ids[k] = assign[lo + k];
+  const uint64_t row = (uint64_t)m * cb, nbytes = (k1 - k0) * row;
+  const uint8_t* src = codes + (lo + k0) * row;
+  uint8_t* dst = p + 4 + 4 * n_d + k0 * row;
+  if ((((uintptr_t)src | (uintptr_t)dst | nbytes) & 3) == 0) {
+    const uint32_t* s4 = reinterpret_cast<const uint32_t*>(src);
+    uint32_t* d4 = reinterpret_cast<uint32_t*>(dst);
+    for (uint64_t q = lane; q < nbytes / 4; q += 64) d4[q] = s4[q];
+  } else {
+    for (uint64_t q = lane; q < nbytes; q += 64) dst[q] = src[q];
+  }
+  if (k1 < n_d) return;
+  const uint64_t total = doc_bytes(n_d, m, cb);
+  for (uint64_t q = 4 + 4 * n_d + n_d * row + lane; q < total; q += 64) p[q] = 0;
 }
 
-// One wave per document (grid-stride): n_d, the centroid ids and the codes,
-// then zero padding.  Doc starts are 8-aligned, so the id array is 4-aligned;
-// codes are copied as 32-bit words when source and destination allow.
+// Phase 3: adds each scan block's carry-in to the document's offset and writes
+// the layouts, one wave per document or slice (grid-stride).
 __global__ __launch_bounds__(256) void doc_write_kernel(
     const uint64_t* __restrict__ doc_offsets, uint64_t n_docs, const uint32_t* __restrict__ assign,
     const uint8_t* __restrict__ codes, uint32_t m, uint32_t cb,
-    const uint64_t* __restrict__ doc_index, uint8_t* __restrict__ payload) {
+    const uint64_t* __restrict__ sums, uint64_t* __restrict__ doc_index,
+    uint8_t* __restrict__ payload, const DocState* __restrict__ st,
+    const DocSlice* __restrict__ slices) {
   const uint32_t lane = threadIdx.x % 64;
   const uint64_t waves = (uint64_t)gridDim.x * (blockDim.x / 64);
-  for (uint64_t d = (uint64_t)blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64; d < n_docs;
-       d += waves) {
+  const uint64_t wave = (uint64_t)blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64;
+  const bool go = st->go != 0;
+  const uint64_t n_slices = go ? st->slices : 0;
+  for (uint64_t i = wave; i < n_slices; i += waves) {
+    const DocSlice sl = slices[i];
+    const uint64_t lo = doc_offsets[sl.doc], n_d = doc_offsets[sl.doc + 1] - lo;
+    const uint64_t k1 = n_d - sl.first < kDocSlice ? n_d : sl.first + kDocSlice;
+    doc_copy(lane, lo, n_d, sl.first, k1,
+             payload + sl.at + sums[sl.doc / (kScanBlock * kScanPer)], assign, codes, m, cb);
+  }
+  for (uint64_t d = wave; d < n_docs; d += waves) {
     const uint64_t lo = doc_offsets[d], n_d = doc_offsets[d + 1] - lo;
-    uint8_t* p = payload + doc_index[d];
-    uint32_t* ids = reinterpret_cast<uint32_t*>(p + 4);
-    if (lane == 0) *reinterpret_cast<uint32_t*>(p) = (uint32_t)n_d;
-    for (uint64_t k = lane; k < n_d; k += 64) ids[k] = assign[lo + k];
-    const uint64_t nbytes = n_d * m * cb;
-    const uint8_t* src = codes + lo * m * cb;
-    uint8_t* dst = p + 4 + 4 * n_d;
-    if (((uintptr_t)src & 3) == 0 && (nbytes & 3) == 0) {
-      const uint32_t* s4 = reinterpret_cast<const uint32_t*>(src);
-      uint32_t* d4 = reinterpret_cast<uint32_t*>(dst);
-      for (uint64_t q = lane; q < nbytes / 4; q += 64) d4[q] = s4[q];
-    } else {
-      for (uint64_t q = lane; q < nbytes; q += 64) dst[q] = src[q];
-    }
-    const uint64_t used = 4 + 4 * n_d + nbytes;
-    const uint64_t total = doc_bytes(n_d, m, cb);
-    for (uint64_t q = used + lane; q < total; q += 64) p[q] = 0;
+    const uint64_t at = doc_index[d] + sums[d / (kScanBlock * kScanPer)];
+    if (lane == 0) doc_index[d] = at;
+    if (go && n_d <= kDocSlice)
+      doc_copy(lane, lo, n_d, 0, n_d, payload + at, assign, codes, m, cb);
   }
 }
 

@@ -98,7 +98,7 @@ struct DeviceState {
   // training / encode workspace
   Buffer xs, codes, e, hist, counts, start, sorted, flags, scal, trace, io_in, io_out, io_cb,
       io_init, counter, kpp_state, kpp_w, kpp_bsum, kpp_bad, status, io_aux, io_out2, scan_sums,
-      io_x1, io_x2, io_x3, crc_tables, fold_pre, fold_chunks, cand_nbr, cand_defer, cand_count, cand_anchor, cand_grid, kpp_src,
+      io_x1, io_x2, io_x3, crc_tables, doc_state, doc_slices, fold_pre, fold_chunks, cand_nbr, cand_defer, cand_count, cand_anchor, cand_grid, kpp_src,
       fold_order, cell_par, cell_cids, cell_ccnt, cell_rec, cell_list;
   // token-aware clustering
   Buffer tac_v, tac_idx, tac_offs, tac_G, tac_spreads, tac_w, tac_e, tac_code, tac_sorted,
@@ -1788,7 +1788,7 @@ int tac_gpu_release_workspace(void) {
                     &ds->io_in,     &ds->io_out,  &ds->io_cb,     &ds->io_init,  &ds->counter,
                     &ds->kpp_state, &ds->kpp_w,   &ds->kpp_bsum,  &ds->kpp_bad,  &ds->status,
                     &ds->io_aux,    &ds->io_out2, &ds->scan_sums, &ds->io_x1,    &ds->io_x2,
-                    &ds->io_x3,     &ds->crc_tables, &ds->fold_pre,  &ds->fold_chunks,
+                    &ds->io_x3,     &ds->crc_tables, &ds->doc_state, &ds->doc_slices, &ds->fold_pre,  &ds->fold_chunks,
                     &ds->tac_v,     &ds->tac_idx, &ds->tac_offs,  &ds->tac_G,
                     &ds->tac_spreads, &ds->tac_w, &ds->tac_e,     &ds->tac_code,
                     &ds->tac_sorted, &ds->tac_tsum, &ds->tac_hist, &ds->tac_counts,
@@ -2307,9 +2307,6 @@ int doc_layouts_core(DeviceState &ds, hipStream_t s, const uint64_t *d_off, uint
                      uint64_t n_tokens, const uint32_t *d_assign, const uint8_t *d_codes,
                      uint32_t m, uint32_t cb, uint64_t *d_index, uint8_t *d_payload,
                      uint64_t payload_len, uint64_t *total_out) {
-  uint32_t *status = nullptr;
-  int st = status_begin(ds, s, &status);
-  if (st) return st;
   if (n_docs == 0) {
     HIP_TRY(hipMemsetAsync(d_index, 0, sizeof(uint64_t), s));
     HIP_TRY(hipStreamSynchronize(s));
@@ -2319,27 +2316,41 @@ int doc_layouts_core(DeviceState &ds, hipStream_t s, const uint64_t *d_off, uint
   const uint64_t per = (uint64_t)kScanBlock * kScanPer;
   const uint64_t nb = (n_docs + per - 1) / per;
   if (nb > 0x7FFFFFFFull) return TAC_ERR_UNSUPPORTED;
-  if ((st = ensure(ds, ds.scan_sums, (size_t)nb * sizeof(uint64_t)))) return st;
+  int st;
+  if ((st = host_words(ds)) || (st = ensure(ds, ds.scan_sums, (size_t)nb * sizeof(uint64_t))) ||
+      (st = ensure(ds, ds.doc_slices, (size_t)doc_slices_most(n_tokens) * sizeof(DocSlice))))
+    return st;
+  if (!ds.doc_state.ptr) {
+    if ((st = ensure(ds, ds.doc_state, sizeof(DocState)))) return st;
+    HIP_TRY(hipMemsetAsync(ds.doc_state.ptr, 0, sizeof(DocState), s));
+  }
   uint64_t *sums = as<uint64_t>(ds.scan_sums);
+  DocState *state = as<DocState>(ds.doc_state);
+  DocSlice *slices = as<DocSlice>(ds.doc_slices);
+  // The three kernels run back to back: the second decides on the device
+  // whether the third writes, and leaves the total in the host words.
   doc_sizes_scan_kernel<<<(unsigned)nb, kScanBlock, 0, s>>>(d_off, n_docs, n_tokens, m, cb,
-                                                           d_index, sums, status);
-  doc_sums_scan_kernel<<<1, kScanBlock, 0, s>>>(sums, (uint32_t)nb, d_index, n_docs);
-  doc_scan_add_kernel<<<(unsigned)nb, kScanBlock, 0, s>>>(d_index, sums, n_docs);
-  LAUNCH_TRY("doc layout scan");
-  uint64_t total = 0;
-  HIP_TRY(hipMemcpyAsync(&total, d_index + n_docs, sizeof(total), hipMemcpyDeviceToHost, s));
-  if ((st = status_collect(ds, s))) return st;  // synchronises the stream
+                                                           d_index, sums, state, slices);
+  doc_sums_scan_kernel<<<1, kScanBlock, 0, s>>>(sums, (uint32_t)nb, d_index, n_docs, payload_len,
+                                                state, ds.host_words);
+  const uint64_t waves_wanted =
+      std::min<uint64_t>(std::max(n_docs, doc_slices_most(n_tokens)), 1ull << 20);
+  const unsigned blocks = (unsigned)((waves_wanted + 3) / 4);
+  doc_write_kernel<<<blocks, 256, 0, s>>>(d_off, n_docs, d_assign, d_codes, m, cb, sums, d_index,
+                                          d_payload, state, slices);
+  LAUNCH_TRY("doc layout kernels");
+  HIP_TRY(hipStreamSynchronize(s));
+  const uint32_t *host = ds.host_words;
+  if (__atomic_load_n(host, __ATOMIC_ACQUIRE)) {
+    g_last_error = "input holds a centroid id or code out of range";
+    return TAC_ERR_INVALID_ARGUMENT;
+  }
+  const uint64_t total = (uint64_t)host[2] << 32 | host[1];
   *total_out = total;
   if (total > payload_len) {
     g_last_error = "payload buffer smaller than the document layouts";
     return TAC_ERR_BUFFER_TOO_SMALL;
   }
-  const uint64_t waves_wanted = n_docs < (1ull << 20) ? n_docs : (1ull << 20);
-  const unsigned blocks = (unsigned)((waves_wanted + 3) / 4);
-  doc_write_kernel<<<blocks, 256, 0, s>>>(d_off, n_docs, d_assign, d_codes, m, cb, d_index,
-                                          d_payload);
-  LAUNCH_TRY("doc_write_kernel");
-  HIP_TRY(hipStreamSynchronize(s));
   return TAC_OK;
 }
 
