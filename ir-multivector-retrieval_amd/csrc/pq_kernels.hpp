@@ -1403,6 +1403,60 @@ __global__ __launch_bounds__(kBlock) void encode_kernel(
   flush_rescans(mine, &lcount, rescans);
 }
 
+// PQ.encode of few rows: LPV lanes share a vector's scan, lane l taking the
+// codewords l, l + LPV, ... by the reference distance, and merge their
+// (distance, index) minima.  PQ.encode's scan starts from +inf with a strict
+// <, so a distance of +inf or NaN never wins and a row without any smaller
+// one gets code 0: the minimum of (distance bits, index) over the distances
+// below +inf, or (+inf, 0).
+//
+// Bound by latency (launch, codebook and row loads, one scan of K / LPV
+// codewords): with eight vectors a thread one block of 2,048 rows per
+// subspace left 180 rows of m32 on 32 blocks, each thread scanning all 256
+// codewords: 39 us a call against 7.3 with this kernel.
+template <int D, int LPV, typename CodeT>
+__global__ __launch_bounds__(kBlock) void encode_small_kernel(
+    const float* __restrict__ x, const float* __restrict__ cb, CodeT* __restrict__ codes,
+    uint64_t n, uint32_t dim, uint32_t M, uint32_t K) {
+  constexpr int DP = Pad<D>::value;
+  constexpr uint32_t kRows = kBlock / LPV;
+  extern __shared__ __attribute__((aligned(16))) float lcb[];  // [K][DP]
+  const uint32_t m = blockIdx.x % M;
+  const uint64_t i = (uint64_t)(blockIdx.x / M) * kRows + threadIdx.x / LPV;
+  const uint32_t l = threadIdx.x % LPV;
+  const float* src = x + (i < n ? i : n - 1) * dim + (uint64_t)m * D;
+  float xv[D];
+#pragma unroll
+  for (int k = 0; k < D; ++k) xv[k] = src[k];
+  const float* cm = cb + (uint64_t)m * K * D;
+  if constexpr (D == DP) {
+    for (uint32_t f = threadIdx.x; f < K * D; f += kBlock) lcb[f] = cm[f];
+  } else {
+    for (uint32_t f = threadIdx.x; f < K * D; f += kBlock) lcb[f / D * DP + f % D] = cm[f];
+  }
+  __syncthreads();
+  float best = __builtin_inff();
+  uint32_t idx = 0;
+#pragma unroll 4
+  for (uint32_t c = l; c < K; c += LPV) {
+    float cv[D];
+    load_padded<D>(lcb + c * DP, cv);
+    const float d = exact_l2sq<D>(xv, cv);
+    const bool less = d < best;
+    best = less ? d : best;
+    idx = less ? c : idx;
+  }
+#pragma unroll
+  for (int off = 1; off < LPV; off <<= 1) {
+    const float o = __shfl_xor(best, off, kWave);
+    const uint32_t oi = __shfl_xor(idx, off, kWave);
+    const bool take = o < best || (o == best && oi < idx);
+    best = take ? o : best;
+    idx = take ? oi : idx;
+  }
+  if (l == 0 && i < n) codes[i * M + m] = (CodeT)idx;
+}
+
 // PQ.decode (src/index/pq.zig:79-88): out[i][m*D + k] = cb[m][code[i][m]][k].
 // A code >= K raises `status` and yields NaN instead of a read.
 template <typename CodeT>

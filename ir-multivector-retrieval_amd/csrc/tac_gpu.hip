@@ -401,15 +401,16 @@ int event_at(DeviceState &ds, size_t idx, hipEvent_t *out) {
 }
 
 // Device counter of vectors the pruned search resolved by a full reference
-// scan; zeroed per call, added to the profile when measuring.
+// scan; zeroed and added to the profile per call when measuring.
 // Device counters: [0] exact rescans, [1] candidate-path deferrals,
 // [2] candidate-path assignments, [3] cell-list encode subspaces,
 // [4] screen deferrals, [5] screen searches.
 constexpr int kCounters = 6;
-int counter_begin(DeviceState &ds, hipStream_t s, unsigned long long **out) {
+int counter_begin(DeviceState &ds, hipStream_t s, bool clear, unsigned long long **out) {
   int st = ensure(ds, ds.counter, kCounters * sizeof(unsigned long long));
   if (st) return st;
-  HIP_TRY(hipMemsetAsync(ds.counter.ptr, 0, kCounters * sizeof(unsigned long long), s));
+  if (clear)  // read only when measuring; kernels add to them always
+    HIP_TRY(hipMemsetAsync(ds.counter.ptr, 0, kCounters * sizeof(unsigned long long), s));
   *out = reinterpret_cast<unsigned long long *>(ds.counter.ptr);
   return TAC_OK;
 }
@@ -543,6 +544,24 @@ inline bool list_lanes4(uint32_t K) {
 }
 inline uint32_t list_split(uint32_t K) {
   return !list_lanes4(K) ? 0u : K >= 512 ? 0xFFFFFFFFu : 32768u;
+}
+
+// Rows up to which encode_small_kernel serves a call: below the candidate
+// passes' 16,384 at sub-dimensions 1-4 (call times in us, the search of eight
+// vectors a thread | this kernel: m32 dsub 2 K256 at 1 row 33 | 9, 1,000
+// 44 | 11, 16,000 60 | 32; m16 dsub 4 K1024 at 180 rows 120 | 13, 16,000
+// 210 | 76), and to 8,192 at 5-8, where the matrix-core screen takes over
+// (m16 dsub 8 K256 at 180 rows 30 | 12, 1,000 48 | 12, 8,000 67 | 26).
+constexpr uint64_t kEncodeSmallRows = 16384, kEncodeSmallRowsWide = 8192;
+inline bool encode_is_small(uint64_t n, uint32_t D) {
+  return D <= 4 ? n < kEncodeSmallRows : n <= kEncodeSmallRowsWide;
+}
+// Its lanes per vector: 16 while the rows are few for the length of a scan
+// (16 | 4 lanes: m16 dsub 4 K256 at 180 rows 9.9 | 11.5 us, 4,000 15.1 |
+// 13.8; dsub 8 at 1,000 rows 12.2 | 17.5, 8,000 29.4 | 25.9; K1024 at 1,000
+// rows 15.2 | 21.4, 8,000 47.8 | 43.5), else 4.
+inline bool encode_wide_lanes(uint64_t n, uint32_t M, uint32_t K, uint32_t D) {
+  return n * M < 24ull * K * D;
 }
 
 template <int D>
@@ -896,9 +915,26 @@ struct Launch {
                                         n, K, iter, tol, check);
     KT_END();
   }
+  template <int LPV, typename CodeT>
+  static int encode_small(const float *x, const float *cb, CodeT *codes, uint64_t n,
+                          uint32_t dim, uint32_t M, uint32_t K, hipStream_t s) {
+    const uint64_t blocks = (n + kBlock / LPV - 1) / (kBlock / LPV) * M;
+    if (blocks > 0x7FFFFFFFull) return TAC_ERR_UNSUPPORTED;
+    KT("encode_small_kernel<%d, %d, %s>", D, LPV, code_name<CodeT>());
+    encode_small_kernel<D, LPV, CodeT><<<(unsigned)blocks, kBlock,
+                                         (size_t)K * Pad<D>::value * sizeof(float), s>>>(
+        x, cb, codes, n, dim, M, K);
+    KT_END();
+    return TAC_OK;
+  }
+  // The vector-unit search of n rows that no other pass takes.
   template <typename CodeT>
   static int encode(const float *x, const float *cb, CodeT *codes, uint64_t n, uint32_t dim,
                     uint32_t M, uint32_t K, unsigned long long *rescans, hipStream_t s) {
+    if (encode_is_small(n, D))
+      return encode_wide_lanes(n, M, K, D)
+                 ? encode_small<16, CodeT>(x, cb, codes, n, dim, M, K, s)
+                 : encode_small<4, CodeT>(x, cb, codes, n, dim, M, K, s);
     const uint32_t Kp = (K + kPruneBlock - 1) / kPruneBlock * kPruneBlock;
     const size_t lds = (size_t)Kp * (Pad<D>::value + 1) * sizeof(float) + 2 * sizeof(uint32_t);
     const uint64_t tiles = (n + kBlock * VPT - 1) / (kBlock * VPT);
@@ -1163,9 +1199,9 @@ int train_core(DeviceState &ds, hipStream_t s, const float *d_x, uint64_t n, uin
   HIP_TRY(hipMemsetAsync(done, 0, 3 * M * sizeof(uint32_t), s));
   HIP_TRY(hipMemsetAsync(wcss, 0, 2 * M * sizeof(float), s));
   unsigned long long *rescans = nullptr;
-  if ((st = counter_begin(ds, s, &rescans))) return st;
-
   const bool profile = g_profile;
+  if ((st = counter_begin(ds, s, profile, &rescans))) return st;
+
   ClockScope clock(ds, s);
   size_t ev = 0;
   hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -1499,7 +1535,7 @@ int encode_core(DeviceState &ds, hipStream_t s, const float *d_x, uint64_t n, ui
   hipEvent_t a = nullptr, b = nullptr;
   int st;
   unsigned long long *rescans = nullptr;
-  if ((st = counter_begin(ds, s, &rescans))) return st;
+  if ((st = counter_begin(ds, s, profile, &rescans))) return st;
   if (profile) {
     if ((st = event_at(ds, 0, &a)) || (st = event_at(ds, 1, &b))) return st;
     HIP_TRY(hipEventRecord(a, s));
@@ -1570,7 +1606,8 @@ int encode_core(DeviceState &ds, hipStream_t s, const float *d_x, uint64_t n, ui
                                              slices + (size_t)M * n, as<uint32_t>(ds.cand_count),
                                              n, dim, M, K, L, rescans, s));
     }
-  } else if (D >= 5 && D <= 8 && screen_wanted(K) && n <= 0xFFFFFFFFull) {
+  } else if (D >= 5 && D <= 8 && screen_wanted(K) && n <= 0xFFFFFFFFull &&
+             !encode_is_small(n, D)) {
     if ((st = ensure(ds, ds.cand_defer, (size_t)2 * M * n * sizeof(uint32_t))) ||
         (st = ensure(ds, ds.cand_count, (size_t)M * sizeof(uint32_t))))
       return st;
@@ -1973,14 +2010,12 @@ int tac_pq_encode_device_noalloc(const float *d_residuals, uint64_t n, uint32_t 
     off += (bytes + 255) & ~(size_t)255;
     return p;
   };
-  // [0] exact rescans, [1] and [2] stay unused (no profiling here)
+  // where the kernels count rescans; never read, so never cleared
   auto *counters = reinterpret_cast<unsigned long long *>(take(3 * sizeof(unsigned long long)));
-  zero_words_kernel<<<1, kWave, 0, s>>>(reinterpret_cast<uint32_t *>(counters), 6);
-  LAUNCH_TRY("zero_words_kernel");
   // Sub-dimensions 5-8 with ksub <= 256: the matrix-core screen, its
   // deferred list (one word per row and subspace) and count in the scratch,
   // in batches of whole sort tiles that fit.
-  if (D >= 5 && D <= 8 && screen_wanted(ksub)) {
+  if (D >= 5 && D <= 8 && screen_wanted(ksub) && !encode_is_small(n, D)) {
     uint32_t *dcount = reinterpret_cast<uint32_t *>(take((size_t)m * sizeof(uint32_t)));
     const size_t left = off < kNoAllocScratchBytes ? kNoAllocScratchBytes - off : 0;
     uint64_t sb = left / (sizeof(uint32_t) * (size_t)m) / kSortTile * kSortTile;
