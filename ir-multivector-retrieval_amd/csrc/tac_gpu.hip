@@ -98,7 +98,7 @@ struct DeviceState {
   // training / encode workspace
   Buffer xs, codes, e, hist, counts, start, sorted, flags, scal, trace, io_in, io_out, io_cb,
       io_init, counter, kpp_state, kpp_w, kpp_bsum, kpp_bad, status, io_aux, io_out2, scan_sums,
-      io_x1, io_x2, io_x3, crc_tables, doc_state, doc_slices, fold_pre, fold_chunks, cand_nbr, cand_defer, cand_count, cand_anchor, cand_grid, kpp_src,
+      io_x1, io_x2, io_x3, crc_tables, doc_state, doc_slices, fold_pre, fold_chunks, cand_nbr, cand_defer, cand_count, cand_anchor, cand_grid, kpp_src, kpp_patch,
       fold_order, cell_par, cell_cids, cell_ccnt, cell_rec, cell_list;
   // token-aware clustering
   Buffer tac_v, tac_idx, tac_offs, tac_G, tac_spreads, tac_w, tac_e, tac_code, tac_sorted,
@@ -891,11 +891,14 @@ struct Launch {
     KT_END();
     return TAC_OK;
   }
-  static void kpp_update(const float *xs, float *w, uint16_t *src, double *bsum, uint32_t *bad,
-                         const KppState *st, float *cb, uint64_t n, uint32_t M, uint32_t K,
-                         uint32_t c, uint32_t NB, hipStream_t s) {
-    kpp_update_kernel<D><<<dim3(NB, M), kKppThreads, 0, s>>>(xs, w, src, bsum, bad, st, cb, n,
-                                                              K, c, NB);
+  static void kpp_round(const float *xs, float *w, uint16_t *src, double *bsum,
+                        uint64_t bstride, float *patch, uint32_t *bad, const KppSeed *in,
+                        KppSeed *out, float *cb, uint64_t n, uint32_t M, uint32_t K, uint32_t NB,
+                        uint32_t exact_only, hipStream_t s) {
+    auto *kernel = NB * kKppRuns <= kKppFusedRuns ? kpp_round_kernel<D, true>
+                                                  : kpp_round_kernel<D, false>;
+    kernel<<<dim3(NB, M), kKppThreads, 0, s>>>(xs, w, src, bsum, bstride, patch, bad, in, out, cb,
+                                               n, K, NB, exact_only);
   }
   static void fold(const float *sorted, const uint32_t *counts, const uint32_t *start,
                    float *cb, const uint32_t *done, const uint32_t *order, uint64_t n, uint32_t M,
@@ -1007,15 +1010,18 @@ int kmeanspp(DeviceState &ds, hipStream_t s, const SubspaceGroup *groups, uint32
              const float *xs, uint64_t n, uint32_t M, uint32_t K, uint32_t D, uint64_t seed,
              float *cb) {
   const uint32_t NB = (uint32_t)((n + kKppBlock - 1) / kKppBlock);
+  const uint32_t n_runs = NB * kKppRuns;
+  const bool fused = n_runs <= kKppFusedRuns;
   const uint32_t DP = pad_of(D);
   int st;
-  if ((st = ensure(ds, ds.kpp_state, (size_t)M * sizeof(KppState))) ||
+  if ((st = ensure(ds, ds.kpp_state, (size_t)2 * M * sizeof(KppSeed))) ||
       (st = ensure(ds, ds.kpp_w, (size_t)M * n * sizeof(float))) ||
       (st = ensure(ds, ds.kpp_src, (size_t)M * n * sizeof(uint16_t))) ||
-      (st = ensure(ds, ds.kpp_bsum, (size_t)M * NB * sizeof(double))) ||
+      (st = ensure(ds, ds.kpp_bsum, (size_t)2 * M * n_runs * sizeof(double))) ||
+      (st = ensure(ds, ds.kpp_patch, (size_t)2 * M * kKppRun * sizeof(float))) ||
       (st = ensure(ds, ds.kpp_bad, (size_t)M * sizeof(uint32_t))))
     return st;
-  // exact weight folds of the fallback: chunk prefixes / start values and
+  // exact weight folds of the pending draws: chunk prefixes / start values and
   // descriptors (the same buffers, and sizes, as the wcss fold of training)
   const uint32_t nfc = (uint32_t)((n + kFoldChunk - 1) / kFoldChunk);
   if ((st = ensure(ds, ds.fold_pre, (size_t)M * nfc * sizeof(double))) ||
@@ -1027,46 +1033,71 @@ int kmeanspp(DeviceState &ds, hipStream_t s, const SubspaceGroup *groups, uint32
   // (the same picks, slower; the parallel band test is skipped).
   const char *exact_env = getenv("TAC_GPU_KPP_EXACT");
   const uint32_t exact_only = exact_env != nullptr && exact_env[0] == '1';
-  KppState *state = as<KppState>(ds.kpp_state);
+  KppSeed *state[2] = {as<KppSeed>(ds.kpp_state), as<KppSeed>(ds.kpp_state) + M};
   float *w = as<float>(ds.kpp_w);
+  float *patch = as<float>(ds.kpp_patch);
   uint16_t *src = as<uint16_t>(ds.kpp_src);
   double *bsum = as<double>(ds.kpp_bsum);
   uint32_t *bad = as<uint32_t>(ds.kpp_bad);
-  auto launch_all = [&]() -> int {
-    for (uint32_t h = 0; h < H; ++h) {
-      const SubspaceGroup &g = groups[h];
-      kpp_init_kernel<<<(g.Mh + 63) / 64, 64, 0, g.s>>>(state + g.m0, bad + g.m0, seed + g.m0,
-                                                       n, g.Mh);
-      LAUNCH_TRY("kpp_init_kernel");
-    }
-    for (uint32_t c = 0; c < K; ++c) {
+  uint32_t launch = 0;  // the next launch reads state[launch & 1]
+  auto exact = [&](const SubspaceGroup &g) -> int {
+    kpp_exact_kernel<<<g.Mh, kKppFallbackThreads, 0, g.s>>>(
+        w + (uint64_t)g.m0 * n, state[launch & 1] + g.m0, n, fold_pre + (uint64_t)g.m0 * nfc,
+        fold_chunks + (uint64_t)g.m0 * nfc, nfc);
+    LAUNCH_TRY("kpp_exact_kernel");
+    return TAC_OK;
+  };
+  auto rounds = [&](uint32_t count) -> int {
+    for (uint32_t c = 0; c < count; ++c, ++launch) {
       for (uint32_t h = 0; h < H; ++h) {
         const SubspaceGroup &g = groups[h];
         const uint64_t m0 = g.m0;
-        DISPATCH_D(D, kpp_update(xs + m0 * n * DP, w + m0 * n, src + m0 * n, bsum + m0 * NB,
-                                 bad + m0, state + m0, cb + m0 * K * D, n, g.Mh, K, c, NB, g.s));
-        LAUNCH_TRY("kpp_update_kernel");
-        if (c + 1 == K) continue;
-        kpp_select_kernel<<<g.Mh, 1024, 0, g.s>>>(w + m0 * n, bsum + m0 * NB, bad + m0,
-                                                  state + m0, n, NB, exact_only);
-        LAUNCH_TRY("kpp_select_kernel");
-        kpp_fallback_kernel<<<g.Mh, kKppFallbackThreads, 0, g.s>>>(
-            w + m0 * n, state + m0, n, fold_pre + m0 * nfc, fold_chunks + m0 * nfc, nfc);
-        LAUNCH_TRY("kpp_fallback_kernel");
+        if (!fused && launch > 0) {
+          kpp_draw_kernel<<<g.Mh, kKppFallbackThreads, 0, g.s>>>(
+              w + m0 * n, bsum + m0 * n_runs, (uint64_t)M * n_runs, bad + m0,
+              state[launch & 1] + m0, n, K, n_runs, exact_only, fold_pre + m0 * nfc,
+              fold_chunks + m0 * nfc, nfc);
+          LAUNCH_TRY("kpp_draw_kernel");
+        }
+        DISPATCH_D(D, kpp_round(xs + m0 * n * DP, w + m0 * n, src + m0 * n,
+                                bsum + m0 * n_runs, (uint64_t)M * n_runs,
+                                patch + m0 * 2 * kKppRun, bad + m0, state[launch & 1] + m0,
+                                state[~launch & 1] + m0, cb + m0 * K * D, n, g.Mh, K, NB,
+                                exact_only, g.s));
+        LAUNCH_TRY("kpp_round_kernel");
       }
     }
     return TAC_OK;
   };
-  st = launch_all();
-  // The call's stream waits for the other groups, also after an error.
-  for (uint32_t h = 1; h < H; ++h) {
-    HIP_TRY(hipEventRecord(ds.aux_join[h - 1], groups[h].s));
-    HIP_TRY(hipStreamWaitEvent(s, ds.aux_join[h - 1], 0));
+  auto init = [&]() -> int {
+    for (uint32_t h = 0; h < H; ++h) {
+      const SubspaceGroup &g = groups[h];
+      kpp_init_kernel<<<(g.Mh + 63) / 64, 64, 0, g.s>>>(state[0] + g.m0, bad + g.m0, seed + g.m0,
+                                                       n, g.Mh);
+      LAUNCH_TRY("kpp_init_kernel");
+    }
+    return TAC_OK;
+  };
+  std::vector<KppSeed> hs(M);
+  st = init();
+  for (uint32_t left = K; left > 0;) {
+    if (!st) st = rounds(exact_only && fused ? std::min(left, 2u) : left);
+    // The call's stream waits for the other groups, also after an error.
+    for (uint32_t h = 1; h < H; ++h) {
+      HIP_TRY(hipEventRecord(ds.aux_join[h - 1], groups[h].s));
+      HIP_TRY(hipStreamWaitEvent(s, ds.aux_join[h - 1], 0));
+    }
+    if (st) return st;
+    HIP_TRY(hipMemcpyAsync(hs.data(), state[launch & 1], M * sizeof(KppSeed),
+                           hipMemcpyDeviceToHost, s));
+    HIP_TRY(hipStreamSynchronize(s));
+    // Subspaces with a pending draw: the exact draws, then the rounds they
+    // missed (the others pass).
+    left = 0;
+    for (uint32_t m = 0; m < M; ++m)
+      if (!hs[m].err) left = std::max(left, K - hs[m].next);
+    for (uint32_t h = 0; left && h < H && !st; ++h) st = exact(groups[h]);
   }
-  if (st) return st;
-  std::vector<KppState> hs(M);
-  HIP_TRY(hipMemcpyAsync(hs.data(), state, M * sizeof(KppState), hipMemcpyDeviceToHost, s));
-  HIP_TRY(hipStreamSynchronize(s));
   for (uint32_t m = 0; m < M; ++m)
     if (hs[m].err) return hs[m].err;
   return TAC_OK;
@@ -1835,7 +1866,7 @@ int tac_gpu_release_workspace(void) {
                     &ds->tac_probs, &ds->tac_tiles, &ds->tac_chl, &ds->tac_cprob,
                     &ds->tac_inv,   &ds->tac_rsum, &ds->tac_ranges, &ds->cand_nbr,
                     &ds->cand_defer, &ds->cand_count, &ds->cand_anchor, &ds->cand_grid,
-                    &ds->kpp_src,   &ds->fold_order, &ds->tac_h, &ds->tac_ktiles,
+                    &ds->kpp_src,   &ds->kpp_patch, &ds->fold_order, &ds->tac_h, &ds->tac_ktiles,
                     &ds->tac_big};
   for (Buffer *b : bufs) {
     if (b->ptr) HIP_TRY(hipFree(b->ptr));
