@@ -1177,6 +1177,178 @@ __device__ inline Acc fold_apply_wave(const float* __restrict__ em, uint64_t n,
   return s;
 }
 
+// fold_apply_wave for an fp32 fold by a block of kBlock threads, which first
+// stages, a window of kFoldWindow chunks at a time, each chunk's quantized sum
+// for the binade of its approximate start `pre` (candidate 1 of its
+// descriptor) and the terms of the chunks that will not fit: those without a
+// clean sum and those whose approximate start and end lie in different
+// binades.  Wave 0 then applies the window out of LDS; a chunk whose start
+// lies in another binade than `pre` told, and one that does not fit where
+// `pre` did not tell, is added from its terms (read from memory if they are
+// not staged): a prediction costs time when it fails, the sum is the serial
+// one.
+//
+// Bound by the serial adds of the chunks that do not fit (about 20 a fold,
+// 256 adds of a dependent chain each) and by latency: a wave by itself waited
+// for memory twice a chunk, 61 us a fold of 117,645 terms; 36 now.
+// Inclusive prefix sum of u32 over the wave's lanes (wave_inclusive_sum_u64).
+__device__ __forceinline__ uint32_t wave_inclusive_sum_u32(uint32_t v) {
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, true);
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, true);
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, true);
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, true);
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, true);
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, true);
+  return v;
+}
+__device__ __forceinline__ float readlane_f32(float v, uint32_t l) {
+  return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(v), (int)l));
+}
+
+// s plus the kFoldChunk terms in LDS at `buf` (zero past the fold's end), in
+// order, by one wave.  Four terms a lane: while s is normal, one prefix sum of
+// the lanes' quantized sums adds the lanes up to the first whose terms do not
+// all fit s's binade, whose four terms are then added one by one.  A chunk
+// that crosses a binade or holds a tie takes two or three such steps; after
+// kFoldSteps, and from a sum that is not normal, the rest is added serially.
+constexpr int kFoldSteps = 3;
+__device__ inline float fold_chunk_terms(float s, const float* buf) {
+  const uint32_t lane = threadIdx.x % kWave;
+  constexpr uint32_t kTop = 2u << FoldTraits<float>::kFrac;  // past the binade, in ulps
+  uint32_t l0 = 0;  // lanes below l0 are added
+  const float4 v4 = reinterpret_cast<const float4*>(buf)[lane];
+  const float v[4] = {v4.x, v4.y, v4.z, v4.w};
+  for (int it = 0; it < kFoldSteps && l0 < kWave && fold_is_normal_positive(s); ++it) {
+    const uint32_t m = (uint32_t)fold_units(s);
+    const int32_t k = fold_exponent(s);
+    uint32_t q = 0;
+    bool ok = true;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint64_t qi = fold_quantize<float>(v[j], k);  // below 2^24 + 1 unless kFoldBad
+      ok = ok && qi != kFoldBad;
+      q += qi == kFoldBad ? 0u : (uint32_t)qi;
+    }
+    const bool mine = lane >= l0;
+    // lanes past the first that does not fit may wrap; they are not looked at
+    const uint32_t P = wave_inclusive_sum_u32(mine && ok ? q : 0u);
+    const uint64_t bad = __ballot(mine && !(ok && m + P < kTop));
+    const uint32_t f = bad ? (uint32_t)__builtin_ctzll(bad) : kWave;
+    if (f > l0) s = fold_with_units(s, m + (uint32_t)__builtin_amdgcn_readlane((int)P, (int)f - 1));
+    if (f < kWave)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) s = s + readlane_f32(v[j], f);
+    l0 = f + 1;
+  }
+#pragma unroll 4
+  for (uint32_t t = l0 * 4; t < kFoldChunk; t += 4) {
+    const float4 x = *reinterpret_cast<const float4*>(buf + t);
+    s = s + x.x;
+    s = s + x.y;
+    s = s + x.z;
+    s = s + x.w;
+  }
+  return s;
+}
+
+constexpr uint32_t kFoldWindow = 1024;
+constexpr uint32_t kFoldStaged = 32;  // chunks whose terms are staged
+
+struct FoldStage {
+  __attribute__((aligned(16))) float terms[kFoldStaged + 1][kFoldChunk];  // the last: unstaged
+  uint32_t q[kFoldWindow];
+  uint8_t binade[kFoldWindow];  // exponent bits of the binade of q; 0: no clean sum
+  uint8_t slot[kFoldWindow];    // row of `terms`, or kFoldStaged
+  uint16_t chunk_of[kFoldStaged];
+  uint32_t n_slots;
+};
+
+__device__ inline float fold_apply_block(const float* __restrict__ em, uint64_t n,
+                                         const FoldChunk* __restrict__ cm,
+                                         const double* __restrict__ pre, uint32_t nc,
+                                         FoldStage& st) {
+  const uint32_t lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
+  float s = 0.0f;
+  for (uint32_t w0 = 0; w0 < nc; w0 += kFoldWindow) {
+    const uint32_t wn = nc - w0 < kFoldWindow ? nc - w0 : kFoldWindow;
+    if (threadIdx.x == 0) st.n_slots = 0;
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < wn; i += kBlock) {
+      const uint32_t j = w0 + i;
+      const float a = (float)pre[j];
+      const float b = j + 1 < nc ? (float)pre[j + 1] : a;
+      const uint64_t q1 = cm[j].q[1];
+      const bool clean = fold_is_normal_positive(a) && (cm[j].clean & 2u) != 0 &&
+                         q1 <= 2ull << FoldTraits<float>::kFrac;
+      st.q[i] = (uint32_t)q1;
+      st.binade[i] = clean ? (uint8_t)(fold_bits(a) >> FoldTraits<float>::kFrac) : 0;
+      uint32_t slot = kFoldStaged;
+      if (!clean || fold_exponent(a) != fold_exponent(b)) {
+        const uint32_t at = atomicAdd(&st.n_slots, 1u);
+        if (at < kFoldStaged) {
+          slot = at;
+          st.chunk_of[at] = (uint16_t)i;
+        }
+      }
+      st.slot[i] = (uint8_t)slot;
+    }
+    __syncthreads();
+    const uint32_t ns = st.n_slots < kFoldStaged ? st.n_slots : kFoldStaged;
+    constexpr uint32_t kRows = kFoldStaged / (kBlock / kWave), kPer = kFoldChunk / kWave;
+    float v[kRows][kPer];  // of the wave's rows, all in flight
+#pragma unroll
+    for (uint32_t r = 0; r < kRows; ++r) {
+      const uint32_t k = w + r * (kBlock / kWave);
+      if (k >= ns) break;
+      const uint32_t j = w0 + st.chunk_of[k], len = fold_chunk_len(n, j);
+      const float* src = em + (uint64_t)j * kFoldChunk;
+#pragma unroll
+      for (uint32_t t = 0; t < kPer; ++t)
+        v[r][t] = t * kWave + lane < len ? src[t * kWave + lane] : 0.0f;
+    }
+#pragma unroll
+    for (uint32_t r = 0; r < kRows; ++r) {
+      const uint32_t k = w + r * (kBlock / kWave);
+      if (k >= ns) break;
+#pragma unroll
+      for (uint32_t t = 0; t < kPer; ++t) st.terms[k][t * kWave + lane] = v[r][t];
+    }
+    __syncthreads();
+    if (w == 0) {
+      for (uint32_t i = 0; i < wn;) {
+        const uint32_t cnt = wn - i < kWave ? wn - i : kWave;
+        uint32_t b = 0;  // chunks applied through the prefix sum
+        if (fold_is_normal_positive(s)) {
+          const uint32_t m = (uint32_t)fold_units(s);
+          uint64_t Q = kFoldBad;
+          if (lane < cnt && st.binade[i + lane] == fold_bits(s) >> FoldTraits<float>::kFrac)
+            Q = st.q[i + lane];
+          const bool ok = Q != kFoldBad;  // then at most 2^24: 64 of them fit 32 bits
+          const uint32_t P = wave_inclusive_sum_u32(ok ? (uint32_t)Q : 0u);
+          const uint64_t bad = __ballot(lane < cnt && !(ok && fold_run_fits<float>(m, P)));
+          b = bad ? (uint32_t)__builtin_ctzll(bad) : cnt;
+          if (b > 0)
+            s = fold_with_units(s, m + (uint32_t)__builtin_amdgcn_readlane((int)P, (int)b - 1));
+        }
+        i += b;
+        if (b < cnt) {
+          const uint32_t j = w0 + i, slot = st.slot[i], len = fold_chunk_len(n, j);
+          if (slot == kFoldStaged) {
+            wave_lds_sync();
+            for (uint32_t t = lane; t < kFoldChunk; t += kWave)
+              st.terms[slot][t] = t < len ? em[(uint64_t)j * kFoldChunk + t] : 0.0f;
+            wave_lds_sync();
+          }
+          s = fold_chunk_terms(s, st.terms[slot]);
+          ++i;
+        }
+      }
+    }
+    __syncthreads();
+  }
+  return s;
+}
+
 // Chunk sums, one wave per chunk, four chunks per block.
 __global__ __launch_bounds__(kBlock) void wcss_chunk_sums_kernel(
     const float* __restrict__ e, double* __restrict__ csum, const uint32_t* __restrict__ done,
@@ -1208,15 +1380,16 @@ __global__ __launch_bounds__(kBlock) void wcss_quantize_kernel(
   fold_quantize_chunk_wave<float>(e + (uint64_t)m * n, n, j, pre[at], chunks + at);
 }
 
-// One wave per subspace applies the chunks in order.
-__global__ __launch_bounds__(kWave) void wcss_apply_kernel(
-    const float* __restrict__ e, const FoldChunk* __restrict__ chunks, float* __restrict__ wcss,
-    const uint32_t* __restrict__ done, uint64_t n, uint32_t nc) {
-  __shared__ __attribute__((aligned(16))) float buf[kFoldChunk];
+// One block per subspace applies the chunks in order.
+__global__ __launch_bounds__(kBlock) void wcss_apply_kernel(
+    const float* __restrict__ e, const FoldChunk* __restrict__ chunks,
+    const double* __restrict__ pre, float* __restrict__ wcss, const uint32_t* __restrict__ done,
+    uint64_t n, uint32_t nc) {
+  __shared__ FoldStage st;
   const uint32_t m = blockIdx.x;
   if (done[m]) return;
-  const float s = fold_apply_wave<float>(e + (uint64_t)m * n, n, chunks + (uint64_t)m * nc, nc,
-                                         buf, static_cast<float*>(nullptr));
+  const float s = fold_apply_block(e + (uint64_t)m * n, n, chunks + (uint64_t)m * nc,
+                                   pre + (uint64_t)m * nc, nc, st);
   if (threadIdx.x == 0) wcss[m] = s;
 }
 

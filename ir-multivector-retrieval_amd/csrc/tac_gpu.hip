@@ -1406,7 +1406,7 @@ int train_core(DeviceState &ds, hipStream_t s, const float *d_x, uint64_t n, uin
                                                                 nfc);
       KT_END();
       KT("wcss_apply_kernel");
-      wcss_apply_kernel<<<Mh, kWave, 0, hs>>>(e_h, chunks_h, wcss + m0, done_h, n, nfc);
+      wcss_apply_kernel<<<Mh, kBlock, 0, hs>>>(e_h, chunks_h, pre_h, wcss + m0, done_h, n, nfc);
       KT_END();
       LAUNCH_TRY("wcss kernels");
     }
