@@ -464,6 +464,14 @@ int host_words(DeviceState &ds) {
   return TAC_OK;
 }
 
+// The first host word after the stream is synchronised, where the kernels
+// raise it on a centroid id or code out of range.
+int host_status(DeviceState &ds) {
+  if (!__atomic_load_n(ds.host_words, __ATOMIC_ACQUIRE)) return TAC_OK;
+  g_last_error = "input holds a centroid id or code out of range";
+  return TAC_ERR_INVALID_ARGUMENT;
+}
+
 uint32_t pad_of(uint32_t d) { return d <= 1 ? 1 : d <= 2 ? 2 : d <= 4 ? 4 : 8; }
 
 uint32_t code_bits(uint32_t K) {
@@ -2276,9 +2284,10 @@ int validate_residuals(uint64_t n, uint32_t dim) {
 int residuals_core(DeviceState &ds, hipStream_t s, const float *v, uint64_t n, uint32_t dim,
                    const float *cent, uint32_t n_cent, const uint32_t *assign, float *out,
                    float *norms) {
-  uint32_t *status = nullptr;
-  int st = status_begin(ds, s, &status);
+  int st = host_words(ds);
   if (st) return st;
+  uint32_t *status = ds.host_words;
+  *status = 0;
   const uint32_t R = residual_rows(dim);
   const uint64_t blocks = (n + R - 1) / R;
   if (blocks > 0x7FFFFFFFull) return TAC_ERR_UNSUPPORTED;
@@ -2299,7 +2308,8 @@ int residuals_core(DeviceState &ds, hipStream_t s, const float *v, uint64_t n, u
                                                                 status, n, dim, n_cent, R);
   LAUNCH_TRY("residual_kernel");
   if (profile) HIP_TRY(hipEventRecord(b, s));
-  if ((st = status_collect(ds, s))) return st;
+  HIP_TRY(hipStreamSynchronize(s));
+  if ((st = host_status(ds))) return st;
   if (profile) {
     float ms = 0.0f;
     HIP_TRY(hipEventElapsedTime(&ms, a, b));
@@ -2417,10 +2427,7 @@ int doc_layouts_core(DeviceState &ds, hipStream_t s, const uint64_t *d_off, uint
   LAUNCH_TRY("doc layout kernels");
   HIP_TRY(hipStreamSynchronize(s));
   const uint32_t *host = ds.host_words;
-  if (__atomic_load_n(host, __ATOMIC_ACQUIRE)) {
-    g_last_error = "input holds a centroid id or code out of range";
-    return TAC_ERR_INVALID_ARGUMENT;
-  }
+  if ((st = host_status(ds))) return st;
   const uint64_t total = (uint64_t)host[2] << 32 | host[1];
   *total_out = total;
   if (total > payload_len) {
