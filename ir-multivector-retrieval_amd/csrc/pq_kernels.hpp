@@ -1644,7 +1644,7 @@ __global__ void decode_kernel(const CodeT* __restrict__ codes, const float* __re
   const uint32_t m = r / D, k = r % D;
   const uint32_t code = codes[i * M + m];
   if (code >= K) {
-    atomicOr(status, 1u);
+    __hip_atomic_store(status, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     out[g] = __builtin_nanf("");
     return;
   }

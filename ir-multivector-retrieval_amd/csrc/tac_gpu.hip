@@ -43,6 +43,7 @@
 #include <condition_variable>
 #include <mutex>
 #include <string>
+#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -115,6 +116,10 @@ struct DeviceState {
   void *stage[kStageBufs] = {};
   hipEvent_t stage_ev[kStageBufs] = {};
   bool stage_pending[kStageBufs] = {};
+  // pinned buffers of large downloads (download_host)
+  static constexpr int kDownBufs = 4;
+  void *down = nullptr;
+  hipEvent_t down_ev[kDownBufs] = {};
   // words of pinned host memory that kernels write results to (host_words)
   uint32_t *host_words = nullptr;
   // measurement
@@ -251,6 +256,93 @@ int upload_host(DeviceState &ds, void *dst, const void *src, size_t bytes, hipSt
   for (int t = 0; t < T; ++t)
     if (cb_status[t] != TAC_OK) return cb_status[t];
   return TAC_OK;
+}
+
+constexpr size_t kDownChunk = 4u << 20;  // most bytes per staged copy back
+constexpr size_t kDownMin = 2u << 20;    // smaller outputs copy to pageable memory directly
+
+// Device-to-host copy of `bytes` into pageable memory, ordered behind the work
+// on s; returns when dst is written.  Large copies pass in chunks through a
+// ring of pinned buffers: kStageThreads host threads each write their share of
+// every chunk to dst (and take its page faults, when dst is fresh memory)
+// while the DMA fetches the next ones.  A chunk costs some 15 us beside its
+// bytes, so there are at least four of at most 4 MB.  Decode of 65,537 rows
+// to 16.8 MB: 620 us a call, 715 with chunks of 1 MB, 1,040 with a
+// hipMemcpyAsync to the same pageable memory, which one thread empties.  With
+// skip, a host word that the kernels before the copy may raise, dst is left
+// alone when it is raised.
+int download_host(DeviceState &ds, void *dst, const void *src, size_t bytes, hipStream_t s,
+                  const uint32_t *skip = nullptr) {
+  if (bytes == 0) return TAC_OK;
+  if (bytes < kDownMin) {
+    if (skip) {
+      HIP_TRY(hipStreamSynchronize(s));
+      if (__atomic_load_n(skip, __ATOMIC_ACQUIRE)) return TAC_OK;
+    }
+    HIP_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
+    HIP_TRY(hipStreamSynchronize(s));
+    return TAC_OK;
+  }
+  constexpr int T = DeviceState::kStageThreads, B = DeviceState::kDownBufs;
+  if (!ds.down) HIP_TRY(hipHostMalloc(&ds.down, B * kDownChunk, hipHostMallocDefault));
+  for (int b = 0; b < B; ++b)
+    if (!ds.down_ev[b]) HIP_TRY(hipEventCreateWithFlags(&ds.down_ev[b], hipEventDisableTiming));
+  const size_t chunk = std::min(kDownChunk, (bytes / B + 65535) / 65536 * 65536);
+  const size_t nch = (bytes + chunk - 1) / chunk;
+  int dev = 0;
+  HIP_TRY(hipGetDevice(&dev));
+  auto fetch = [&](size_t c) -> hipError_t {  // chunk c into buffer c % B
+    const size_t b = c % B, off = c * chunk;
+    const hipError_t e = hipMemcpyAsync(static_cast<char *>(ds.down) + b * kDownChunk,
+                                        static_cast<const char *>(src) + off,
+                                        std::min(bytes - off, chunk), hipMemcpyDeviceToHost, s);
+    return e != hipSuccess ? e : hipEventRecord(ds.down_ev[b], s);
+  };
+  const size_t ahead = std::min<size_t>(nch, B);
+  for (size_t c = 0; c < ahead; ++c) HIP_TRY(fetch(c));
+  std::atomic<size_t> issued{ahead};            // chunks whose event is recorded
+  std::atomic<int> left[DeviceState::kDownBufs];  // threads yet to empty a buffer
+  for (auto &l : left) l = T;
+  std::atomic<int> failed{(int)hipSuccess};
+  auto work = [&](int tid) {
+    hipError_t e = hipSetDevice(dev);
+    for (size_t c = 0; c < nch && e == hipSuccess; ++c) {
+      while (issued.load(std::memory_order_acquire) <= c) {
+        if (failed.load(std::memory_order_acquire) != (int)hipSuccess) return;
+        std::this_thread::yield();
+      }
+      if ((e = hipEventSynchronize(ds.down_ev[c % B])) != hipSuccess) break;
+      if (skip && __atomic_load_n(skip, __ATOMIC_ACQUIRE)) return;
+      const size_t off = c * chunk, len = std::min(bytes - off, chunk);
+      // shares of whole pages
+      const size_t share = (len / T + 4095) / 4096 * 4096;
+      const size_t lo = std::min(len, share * tid);
+      const size_t hi = tid + 1 == T ? len : std::min(len, lo + share);
+      memcpy(static_cast<char *>(dst) + off + lo,
+             static_cast<char *>(ds.down) + c % B * kDownChunk + lo, hi - lo);
+      if (left[c % B].fetch_sub(1, std::memory_order_acq_rel) == 1 && c + B < nch) {
+        // the last to leave the buffer refills it; buffers empty in order
+        left[c % B].store(T, std::memory_order_release);
+        if ((e = fetch(c + B)) == hipSuccess) issued.fetch_add(1, std::memory_order_acq_rel);
+      }
+    }
+    if (e != hipSuccess) failed.store((int)e, std::memory_order_release);
+  };
+  std::vector<std::thread> helpers;
+  helpers.reserve(T);
+  int st = TAC_OK;
+  try {
+    for (int t = 1; t < T; ++t) helpers.emplace_back(work, t);
+  } catch (const std::system_error &) {
+    // no thread to be had: the copy fails as the other allocations do
+    failed.store((int)hipErrorOutOfMemory, std::memory_order_release);
+  }
+  if (failed.load(std::memory_order_acquire) == (int)hipSuccess) work(0);
+  for (auto &h : helpers) h.join();
+  const hipError_t drained = hipStreamSynchronize(s);  // no copy outlives the call
+  if (failed.load() != (int)hipSuccess) st = hip_status("download", (hipError_t)failed.load());
+  if (!st && drained != hipSuccess) st = hip_status("hipStreamSynchronize", drained);
+  return st;
 }
 
 // Order this call after the previous one that used the workspace.
@@ -426,27 +518,6 @@ int counter_collect(DeviceState &ds, hipStream_t s) {
   g_prof.cell_subspaces += v[3];
   g_prof.screen_deferred += v[4];
   g_prof.screen_vectors += v[5];
-  return TAC_OK;
-}
-
-// Device word that kernels raise on invalid input (a centroid id or code out
-// of range); cleared before the launch, read back after it.
-int status_begin(DeviceState &ds, hipStream_t s, uint32_t **out) {
-  int st = ensure(ds, ds.status, sizeof(uint32_t));
-  if (st) return st;
-  HIP_TRY(hipMemsetAsync(ds.status.ptr, 0, sizeof(uint32_t), s));
-  *out = reinterpret_cast<uint32_t *>(ds.status.ptr);
-  return TAC_OK;
-}
-
-int status_collect(DeviceState &ds, hipStream_t s) {
-  uint32_t v = 0;
-  HIP_TRY(hipMemcpyAsync(&v, ds.status.ptr, sizeof(v), hipMemcpyDeviceToHost, s));
-  HIP_TRY(hipStreamSynchronize(s));
-  if (v) {
-    g_last_error = "input holds a centroid id or code out of range";
-    return TAC_ERR_INVALID_ARGUMENT;
-  }
   return TAC_OK;
 }
 
@@ -1891,6 +1962,12 @@ int tac_gpu_release_workspace(void) {
     b->ptr = nullptr;
     b->bytes = 0;
   }
+  if (ds->down) HIP_TRY(hipHostFree(ds->down));
+  ds->down = nullptr;
+  for (hipEvent_t &e : ds->down_ev) {
+    if (e) HIP_TRY(hipEventDestroy(e));
+    e = nullptr;
+  }
   if (ds->host_words) HIP_TRY(hipHostFree(ds->host_words));
   ds->host_words = nullptr;
   for (int b = 0; b < DeviceState::kStageBufs; ++b) {
@@ -2162,8 +2239,7 @@ int tac_pq_encode(const float *residuals, uint64_t n, uint32_t dim, uint32_t m, 
   if ((st = encode_core(*ds, s, as<float>(ds->io_in), n, dim, m, ksub, as<float>(ds->io_cb),
                         ds->io_out.ptr)))
     return st;
-  HIP_TRY(hipMemcpyAsync(codes_out, ds->io_out.ptr, code_bytes, hipMemcpyDeviceToHost, s));
-  HIP_TRY(hipStreamSynchronize(s));
+  if ((st = download_host(*ds, codes_out, ds->io_out.ptr, code_bytes, s))) return st;
   return end_call(*ds, s);
 }
 
@@ -2190,8 +2266,9 @@ int tac_pq_decode(const void *codes, uint64_t n, uint32_t dim, uint32_t m, uint3
     return st;
   HIP_TRY(hipMemcpyAsync(ds->io_in.ptr, codes, code_bytes, hipMemcpyHostToDevice, s));
   HIP_TRY(hipMemcpyAsync(ds->io_cb.ptr, codebooks, cb_bytes, hipMemcpyHostToDevice, s));
-  uint32_t *status = nullptr;
-  if ((st = status_begin(*ds, s, &status))) return st;
+  if ((st = host_words(*ds))) return st;
+  uint32_t *status = ds->host_words;
+  *status = 0;
   const uint64_t total = n * dim;
   const unsigned blocks = (unsigned)((total + 255) / 256);
   if (ksub <= 256)
@@ -2201,9 +2278,9 @@ int tac_pq_decode(const void *codes, uint64_t n, uint32_t dim, uint32_t m, uint3
     decode_kernel<uint16_t><<<blocks, 256, 0, s>>>(as<uint16_t>(ds->io_in), as<float>(ds->io_cb),
                                                    as<float>(ds->io_out), status, n, m, ksub, D);
   LAUNCH_TRY("decode_kernel");
-  if ((st = status_collect(*ds, s))) return st;
-  HIP_TRY(hipMemcpyAsync(out, ds->io_out.ptr, out_bytes, hipMemcpyDeviceToHost, s));
-  HIP_TRY(hipStreamSynchronize(s));
+  if ((st = download_host(*ds, out, ds->io_out.ptr, out_bytes, s, status)) ||
+      (st = host_status(*ds)))
+    return st;
   return end_call(*ds, s);
 }
 
@@ -2374,10 +2451,9 @@ int tac_residuals(const float *vectors, uint64_t n, uint32_t dim, const float *c
                            n_centroids, as<uint32_t>(ds->io_aux), as<float>(ds->io_out),
                            as<float>(ds->io_out2))))
     return st;
-  HIP_TRY(hipMemcpyAsync(residuals_out, ds->io_out.ptr, x_bytes, hipMemcpyDeviceToHost, s));
-  HIP_TRY(hipMemcpyAsync(norms_out, ds->io_out2.ptr, (size_t)n * sizeof(float),
-                         hipMemcpyDeviceToHost, s));
-  HIP_TRY(hipStreamSynchronize(s));
+  if ((st = download_host(*ds, residuals_out, ds->io_out.ptr, x_bytes, s)) ||
+      (st = download_host(*ds, norms_out, ds->io_out2.ptr, (size_t)n * sizeof(float), s)))
+    return st;
   return end_call(*ds, s);
 }
 
@@ -2660,8 +2736,8 @@ int tac_write_doc_layouts(const uint64_t *doc_offsets, uint64_t n_docs, uint64_t
                              as<uint64_t>(ds->io_x2), as<uint8_t>(ds->io_out), need + 8, &total)))
     return st;
   HIP_TRY(hipMemcpyAsync(doc_index_out, ds->io_x2.ptr, off_b, hipMemcpyDeviceToHost, s));
-  if (total) HIP_TRY(hipMemcpyAsync(payload_out, ds->io_out.ptr, total, hipMemcpyDeviceToHost, s));
   HIP_TRY(hipStreamSynchronize(s));
+  if ((st = download_host(*ds, payload_out, ds->io_out.ptr, total, s))) return st;
   return end_call(*ds, s);
 }
 
