@@ -561,12 +561,21 @@ __global__ __launch_bounds__(kBlock) void scan_apply_kernel(
   const uint32_t c0 = threadIdx.x * per_c;
   const uint32_t nq = c0 < K ? (K - c0 < per_c ? K - c0 : per_c) : 0u;
   uint32_t tot[4] = {0, 0, 0, 0}, before[PER] = {};
-  for (uint32_t gg = 0; gg < G; ++gg)
+  // All ranges' sums are loaded before the first is added: one after another,
+  // the ranges were up to 32 round trips (10.8 us at 58 tiles of 8 subspaces,
+  // 4.9 now).
+  uint32_t sum[kScanRanges][PER];
+#pragma unroll
+  for (uint32_t gg = 0; gg < kScanRanges; ++gg)
+#pragma unroll
+    for (uint32_t q = 0; q < PER; ++q)
+      sum[gg][q] = gg < G && q < nq ? pm[(uint64_t)gg * K + c0 + q] : 0u;
+#pragma unroll
+  for (uint32_t gg = 0; gg < kScanRanges; ++gg)
 #pragma unroll
     for (uint32_t q = 0; q < PER; ++q) {
-      const uint32_t v = q < nq ? pm[(uint64_t)gg * K + c0 + q] : 0u;
-      before[q] += gg < g ? v : 0u;
-      tot[q] += v;
+      before[q] += gg < g ? sum[gg][q] : 0u;
+      tot[q] += sum[gg][q];
     }
   uint32_t local = 0;
 #pragma unroll
