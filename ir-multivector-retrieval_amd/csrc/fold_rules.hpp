@@ -150,6 +150,35 @@ TAC_HD inline uint64_t fold_chunk_q(Acc s, const FoldChunk& ch) {
   return Q > 2 * kOne ? kFoldBad : Q;
 }
 
+// A descriptor of an fp32 fold in 16 bytes of LDS.  A quantized sum above 2^24
+// (alone past the binade) makes its candidate unusable, so the others fit.
+struct FoldSlim {
+  uint32_t q[kFoldCands];
+  uint32_t tag;  // exponent bits of candidate 0; from bit 8 the usable candidates
+};
+constexpr uint32_t kFoldSlimBad = ~0u;
+
+TAC_HD inline FoldSlim fold_slim(const FoldChunk& ch) {
+  using T = FoldTraits<float>;
+  FoldSlim out;
+  uint32_t use = 0;
+  for (int c = 0; c < kFoldCands; ++c) {
+    const bool ok = ((ch.clean >> c) & 1u) != 0 && ch.q[c] <= 2ull << T::kFrac;
+    out.q[c] = (uint32_t)ch.q[c];
+    use |= ok ? 1u << c : 0u;
+  }
+  const int32_t e0 = ch.k0 + T::kBias;  // of a normal start: 0 .. 253
+  out.tag = e0 < 0 || e0 > 255 ? 0u : (uint32_t)e0 | use << 8;
+  return out;
+}
+
+// fold_chunk_q of a normal, positive s; kFoldSlimBad for kFoldBad.
+TAC_HD inline uint32_t fold_slim_q(float s, const FoldSlim& ch) {
+  const uint32_t c = (fold_bits(s) >> FoldTraits<float>::kFrac) - (ch.tag & 0xFFu);
+  if (c >= (uint32_t)kFoldCands || !((ch.tag >> (8 + c)) & 1u)) return kFoldSlimBad;
+  return c == 0 ? ch.q[0] : c == 1 ? ch.q[1] : ch.q[2];
+}
+
 // A run of chunks from s: with P_i the prefix sums of their fold_chunk_q,
 // chunk i adds U * Q_i exactly while fold_units(s) + P_i <= 2^(F+1) - 1, so
 // the run's partial sums are fold_with_units(s, fold_units(s) + P_i) and a

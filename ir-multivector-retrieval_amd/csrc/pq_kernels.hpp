@@ -1203,20 +1203,6 @@ __device__ inline Acc fold_apply_wave(const float* __restrict__ em, uint64_t n,
   return s;
 }
 
-// fold_apply_wave for an fp32 fold by a block of kBlock threads, which first
-// stages, a window of kFoldWindow chunks at a time, each chunk's quantized sum
-// for the binade of its approximate start `pre` (candidate 1 of its
-// descriptor) and the terms of the chunks that will not fit: those without a
-// clean sum and those whose approximate start and end lie in different
-// binades.  Wave 0 then applies the window out of LDS; a chunk whose start
-// lies in another binade than `pre` told, and one that does not fit where
-// `pre` did not tell, is added from its terms (read from memory if they are
-// not staged): a prediction costs time when it fails, the sum is the serial
-// one.
-//
-// Bound by the serial adds of the chunks that do not fit (about 20 a fold,
-// 256 adds of a dependent chain each) and by latency: a wave by itself waited
-// for memory twice a chunk, 61 us a fold of 117,645 terms; 36 now.
 // Inclusive prefix sum of u32 over the wave's lanes (wave_inclusive_sum_u64).
 __device__ __forceinline__ uint32_t wave_inclusive_sum_u32(uint32_t v) {
   v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, true);
@@ -1235,8 +1221,9 @@ __device__ __forceinline__ float readlane_f32(float v, uint32_t l) {
 // order, by one wave.  Four terms a lane: while s is normal, one prefix sum of
 // the lanes' quantized sums adds the lanes up to the first whose terms do not
 // all fit s's binade, whose four terms are then added one by one.  A chunk
-// that crosses a binade or holds a tie takes two or three such steps; after
-// kFoldSteps, and from a sum that is not normal, the rest is added serially.
+// that crosses a binade takes two or three such steps; after kFoldSteps, from a
+// lane that does not fit the binade it leaves the sum in (a tie), and from a sum
+// that is not normal, the rest is added serially.
 constexpr int kFoldSteps = 3;
 __device__ inline float fold_chunk_terms(float s, const float* buf) {
   const uint32_t lane = threadIdx.x % kWave;
@@ -1264,9 +1251,11 @@ __device__ inline float fold_chunk_terms(float s, const float* buf) {
     if (f < kWave)
 #pragma unroll
       for (int j = 0; j < 4; ++j) s = s + readlane_f32(v[j], f);
+    const bool stuck = f == l0 && fold_exponent(s) == k;
     l0 = f + 1;
+    if (stuck) break;
   }
-#pragma unroll 4
+#pragma unroll 8
   for (uint32_t t = l0 * 4; t < kFoldChunk; t += 4) {
     const float4 x = *reinterpret_cast<const float4*>(buf + t);
     s = s + x.x;
@@ -1282,19 +1271,46 @@ constexpr uint32_t kFoldStaged = 32;  // chunks whose terms are staged
 
 struct FoldStage {
   __attribute__((aligned(16))) float terms[kFoldStaged + 1][kFoldChunk];  // the last: unstaged
-  uint32_t q[kFoldWindow];
-  uint8_t binade[kFoldWindow];  // exponent bits of the binade of q; 0: no clean sum
-  uint8_t slot[kFoldWindow];    // row of `terms`, or kFoldStaged
+  __attribute__((aligned(16))) FoldSlim chunk[kFoldWindow];
+  uint8_t slot[kFoldWindow];  // row of `terms`, or kFoldStaged
   uint16_t chunk_of[kFoldStaged];
   uint32_t n_slots;
 };
 
+// fold_apply_wave for an fp32 fold by a block of kBlock threads, which first
+// stages, a window of kFoldWindow chunks at a time, the chunks' descriptors and
+// the terms of the chunks that are expected not to fit: those without a clean
+// sum for the binade of their approximate start `pre`, and those whose
+// approximate start and end lie in different binades.  Wave 0 then applies the
+// window out of LDS.  All three candidate binades are staged: over many terms
+// the serial fp32 sum falls behind the f64 prefix, and its binade is then the
+// one below that of `pre` for thousands of chunks.  A chunk that does not fit
+// where `pre` did not tell is added from its terms in memory: a prediction
+// costs time when it fails, the sum is the serial one.
+//
+// Bound by latency: a prefix step per 64 chunks or binade crossing (about 18
+// crossings a fold), and by the serial adds of chunks with ties.  us a fold by
+// the event timers (which add about 5), one wave of dependent loads | this
+// with the start's binade alone | this: 117,645 chi-square terms 45 | 28 | 30;
+// 60,000,000 of them 2,490 | 28,500 | 2,130; as many equal terms 2,480 |
+// 204,000 | 2,130, and with a tie in every chunk 447,000 | 754,000 | 382,000.
 __device__ inline float fold_apply_block(const float* __restrict__ em, uint64_t n,
                                          const FoldChunk* __restrict__ cm,
                                          const double* __restrict__ pre, uint32_t nc,
                                          FoldStage& st) {
   const uint32_t lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
+  constexpr uint32_t kPer = kFoldChunk / kWave;
   float s = 0.0f;
+  float ahead[kPer];  // wave 0: the terms of chunk `next`
+  uint32_t next = ~0u;
+  auto fetch = [&](uint32_t j) {
+    const uint32_t len = fold_chunk_len(n, j);
+    const float* src = em + (uint64_t)j * kFoldChunk;
+#pragma unroll
+    for (uint32_t t = 0; t < kPer; ++t)
+      ahead[t] = t * kWave + lane < len ? src[t * kWave + lane] : 0.0f;
+    next = j;
+  };
   for (uint32_t w0 = 0; w0 < nc; w0 += kFoldWindow) {
     const uint32_t wn = nc - w0 < kFoldWindow ? nc - w0 : kFoldWindow;
     if (threadIdx.x == 0) st.n_slots = 0;
@@ -1303,11 +1319,9 @@ __device__ inline float fold_apply_block(const float* __restrict__ em, uint64_t 
       const uint32_t j = w0 + i;
       const float a = (float)pre[j];
       const float b = j + 1 < nc ? (float)pre[j + 1] : a;
-      const uint64_t q1 = cm[j].q[1];
-      const bool clean = fold_is_normal_positive(a) && (cm[j].clean & 2u) != 0 &&
-                         q1 <= 2ull << FoldTraits<float>::kFrac;
-      st.q[i] = (uint32_t)q1;
-      st.binade[i] = clean ? (uint8_t)(fold_bits(a) >> FoldTraits<float>::kFrac) : 0;
+      const FoldSlim ch = fold_slim(cm[j]);
+      st.chunk[i] = ch;
+      const bool clean = fold_is_normal_positive(a) && fold_slim_q(a, ch) != kFoldSlimBad;
       uint32_t slot = kFoldStaged;
       if (!clean || fold_exponent(a) != fold_exponent(b)) {
         const uint32_t at = atomicAdd(&st.n_slots, 1u);
@@ -1320,7 +1334,7 @@ __device__ inline float fold_apply_block(const float* __restrict__ em, uint64_t 
     }
     __syncthreads();
     const uint32_t ns = st.n_slots < kFoldStaged ? st.n_slots : kFoldStaged;
-    constexpr uint32_t kRows = kFoldStaged / (kBlock / kWave), kPer = kFoldChunk / kWave;
+    constexpr uint32_t kRows = kFoldStaged / (kBlock / kWave);
     float v[kRows][kPer];  // of the wave's rows, all in flight
 #pragma unroll
     for (uint32_t r = 0; r < kRows; ++r) {
@@ -1346,11 +1360,10 @@ __device__ inline float fold_apply_block(const float* __restrict__ em, uint64_t 
         uint32_t b = 0;  // chunks applied through the prefix sum
         if (fold_is_normal_positive(s)) {
           const uint32_t m = (uint32_t)fold_units(s);
-          uint64_t Q = kFoldBad;
-          if (lane < cnt && st.binade[i + lane] == fold_bits(s) >> FoldTraits<float>::kFrac)
-            Q = st.q[i + lane];
-          const bool ok = Q != kFoldBad;  // then at most 2^24: 64 of them fit 32 bits
-          const uint32_t P = wave_inclusive_sum_u32(ok ? (uint32_t)Q : 0u);
+          const FoldSlim ch = st.chunk[i + (lane < cnt ? lane : 0)];
+          const uint32_t Q = fold_slim_q(s, ch);
+          const bool ok = Q != kFoldSlimBad;  // then at most 2^24: 64 of them fit 32 bits
+          const uint32_t P = wave_inclusive_sum_u32(ok ? Q : 0u);
           const uint64_t bad = __ballot(lane < cnt && !(ok && fold_run_fits<float>(m, P)));
           b = bad ? (uint32_t)__builtin_ctzll(bad) : cnt;
           if (b > 0)
@@ -1358,12 +1371,16 @@ __device__ inline float fold_apply_block(const float* __restrict__ em, uint64_t 
         }
         i += b;
         if (b < cnt) {
-          const uint32_t j = w0 + i, slot = st.slot[i], len = fold_chunk_len(n, j);
+          const uint32_t j = w0 + i, slot = st.slot[i];
           if (slot == kFoldStaged) {
+            // Unexpected chunks come in runs (a long stretch of ties): the
+            // next one's terms are loaded while this one's are added.
+            if (next != j) fetch(j);
             wave_lds_sync();
-            for (uint32_t t = lane; t < kFoldChunk; t += kWave)
-              st.terms[slot][t] = t < len ? em[(uint64_t)j * kFoldChunk + t] : 0.0f;
+#pragma unroll
+            for (uint32_t t = 0; t < kPer; ++t) st.terms[slot][t * kWave + lane] = ahead[t];
             wave_lds_sync();
+            if (j + 1 < nc) fetch(j + 1);
           }
           s = fold_chunk_terms(s, st.terms[slot]);
           ++i;

@@ -118,6 +118,39 @@ static Acc chunked_runs(const std::vector<float>& e, std::vector<Acc>* starts) {
   return s;
 }
 
+// The block fold of fp32 terms: runs of 64 chunks through the 16-byte
+// descriptors.  `terms` counts the chunks added from their terms, `lagging` those
+// whose sum lies in another binade than the f64 prefix that placed the candidates.
+static float block_runs(const std::vector<float>& e, uint64_t* terms, uint64_t* lagging) {
+  const size_t n = e.size();
+  const std::vector<FoldChunk> chs = describe<float>(e);
+  const size_t nc = chs.size();
+  float s = 0;
+  size_t j = 0;
+  while (j < nc) {
+    const size_t cnt = std::min<size_t>(64, nc - j);
+    size_t b = 0;
+    if (fold_is_normal_positive(s)) {
+      const uint32_t m = (uint32_t)fold_units(s);
+      uint32_t P = 0;
+      for (; b < cnt; ++b) {
+        const uint32_t Q = fold_slim_q(s, fold_slim(chs[j + b]));
+        if (Q == kFoldSlimBad || !fold_run_fits<float>(m, P + Q)) break;
+        *lagging += fold_exponent(s) != chs[j + b].k0 + 1;
+        P += Q;
+      }
+      if (b > 0) s = fold_with_units(s, m + P);
+    }
+    j += b;
+    if (b < cnt) {
+      ++*terms;
+      for (size_t i = j * kFoldChunk; i < std::min(n, (j + 1) * kFoldChunk); ++i) s = s + e[i];
+      ++j;
+    }
+  }
+  return s;
+}
+
 // weightedSample after its checks (rng.zig:70-81), given the draw r.
 static size_t sample_serial(const std::vector<float>& w, double r) {
   const double total = serial<double>(w);
@@ -176,6 +209,14 @@ int main() {
       std::printf("MISMATCH f64 %s n=%zu serial=%a chunked=%a\n", what, e.size(), c, d);
       ++bad;
     }
+    {
+      uint64_t terms = 0, lagging = 0;
+      const float s = block_runs(e, &terms, &lagging);
+      if (!same(a, s)) {
+        std::printf("MISMATCH f32 block %s n=%zu serial=%a block=%a\n", what, e.size(), a, s);
+        ++bad;
+      }
+    }
     // runs of 64 chunks, with the chunk starts
     std::vector<float> s32a, s32b;
     std::vector<double> s64a, s64b;
@@ -231,6 +272,19 @@ int main() {
     std::vector<float> g(300000, 0x1p-30f);  // f64 half-ulp ties at 2^23
     g[0] = 0x1p23f;
     run("half-ulp-f64", g);
+  }
+  {
+    // Equal terms round the same way in every step, so the fp32 sum falls
+    // behind the f64 prefix by whole binades' worth of chunks: every one must
+    // still go through its descriptor.  Of these 31,250 chunks 439 lie a binade
+    // behind; the start's binade alone would add 455 from their terms, and a
+    // binade crossing or a start from zero adds one each (16).
+    std::vector<float> e(8000000, 0.49f);
+    uint64_t terms = 0, lagging = 0;
+    const float a = serial<float>(e), b = block_runs(e, &terms, &lagging);
+    std::printf("equal terms: %llu chunks from their terms, %llu a binade behind\n",
+                (unsigned long long)terms, (unsigned long long)lagging);
+    bad += !same(a, b) || lagging < 400 || terms > 32;
   }
   // weightedSample through the chunk starts
   uint64_t fbs = 0;

@@ -58,3 +58,16 @@ def test_term_patterns(gpu, kind):
 def test_convergence_is_the_oracles(gpu):
     x = (np.random.default_rng(8).standard_normal((50_000, 16)) * 0.3).astype(np.float32)
     _check(x, 4, 64, iters=25, tol=1e-3)
+
+
+@pytest.mark.parametrize("n", [1_521_797, 8_000_000])
+def test_sum_a_binade_behind(gpu, n):
+    """Equal terms: the serial fp32 sum falls behind the f64 prefix that places
+    the chunks' candidate binades (88 chunks of 1,521,797 terms, 439 of 8,000,000)."""
+    x = np.full((n, 1), 0.7, np.float32)
+    x[::2] *= -1
+    init = np.zeros((1, 1, 1), np.float32)
+    got = pq.train(x, 1, 0, m=1, ksub=1, max_iters=1, tol=NEVER, init_codebooks=init)
+    ref = orc.pq_train(x, 1, 1, 1, init=init, max_iters=1, tol=NEVER, n_threads=1)
+    assert ref.status == 0
+    assert np.array_equal(got.stats.wcss.view(np.uint32), ref.wcss.view(np.uint32))
