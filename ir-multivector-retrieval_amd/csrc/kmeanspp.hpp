@@ -75,6 +75,12 @@ __device__ __forceinline__ double wave_inclusive_sum_f64(double v) {
 __device__ __forceinline__ double readlane_f64(double v, uint32_t l) {
   return __longlong_as_double((long long)readlane_u64((uint64_t)__double_as_longlong(v), l));
 }
+// The lane below's value (0 in lane 0): exclusive sums from inclusive ones.
+// Inclusive minus own would carry a rounding error of the own value's size,
+// which the bands of kpp_decides, relative to the prefix, do not cover.
+__device__ __forceinline__ double wave_below_f64(double v) {
+  return __longlong_as_double((long long)dpp_u64<0x138, 0xF>((uint64_t)__double_as_longlong(v)));
+}
 
 // What the draw of a round found.
 struct KppDraw {
@@ -92,7 +98,7 @@ constexpr uint32_t kKppFusedRuns = kKppLaneRuns * kWave;
 // The draw from the weights' sums per run and the weights, by one wave; lane l
 // owns the runs from l * per on (per = ceil(n_runs / 64)).  FUSED: n_runs is
 // at most kKppFusedRuns; else `share` is the lane's total.  The bands of
-// kpp_decides hold for sums in any order.
+// kpp_decides hold for sums in any order, formed by additions only.
 template <bool FUSED>
 __device__ __forceinline__ KppDraw kpp_draw_wave(const double* __restrict__ sums, uint32_t n_runs,
                                                  double share, const float* wm,
@@ -124,7 +130,7 @@ __device__ __forceinline__ KppDraw kpp_draw_wave(const double* __restrict__ sums
   const uint32_t fl = (uint32_t)__builtin_ctzll(over);
   // the run within that lane's share (its last when rounding leaves none)
   const uint32_t f0 = fl * per, f1 = f0 + per < n_runs ? f0 + per : n_runs;
-  double before = readlane_f64(incl - share, fl);
+  double before = fl ? readlane_f64(incl, fl - 1) : 0.0;
   uint32_t run = f0;
   if constexpr (FUSED) {
 #pragma unroll
@@ -137,13 +143,14 @@ __device__ __forceinline__ KppDraw kpp_draw_wave(const double* __restrict__ sums
   } else {
     for (uint32_t base = f0;; base += kWave) {
       const double x = base + lane < f1 ? sums[base + lane] : 0.0;
-      const double end = before + wave_inclusive_sum_f64(x);
+      const double within = wave_inclusive_sum_f64(x);
+      const double end = before + within;
       const uint32_t last = f1 - 1 - base < kWave ? f1 - 1 - base : kWave - 1;
       const uint64_t in = __ballot(base + lane < f1 && u < end);
       if (in || base + kWave >= f1) {
         const uint32_t at = in ? (uint32_t)__builtin_ctzll(in) : last;
         run = base + at;
-        before = readlane_f64(end - x, at);
+        before = before + (at ? readlane_f64(within, at - 1) : 0.0);
         break;
       }
       before = readlane_f64(end, kWave - 1);
@@ -161,7 +168,7 @@ __device__ __forceinline__ KppDraw kpp_draw_wave(const double* __restrict__ sums
   }
 #pragma unroll
   for (uint32_t q = 0; q < kPer; ++q) sum += v[q];
-  double p = before + (wave_inclusive_sum_f64(sum) - sum), prev = p, at = p;
+  double p = before + wave_below_f64(wave_inclusive_sum_f64(sum)), prev = p, at = p;
   uint32_t k = kKppNone;
 #pragma unroll
   for (uint32_t q = 0; q < kPer; ++q) {

@@ -5,9 +5,14 @@
 //   2. whenever kpp_decides() accepts a candidate computed from prefix sums
 //      in a different summation order, it is the index the reference's
 //      sequential f64 weightedSample (src/util/rng.zig:57-82) returns —
-//      including draws aimed at the cumulative boundaries themselves.
+//      including draws aimed at the cumulative boundaries themselves;
+//   3. the same of the seeding kernels' own sums (lanes' shares of the runs,
+//      the wave's prefix sums by row shifts and broadcasts), where a weight far
+//      larger than all before it sits in the drawn share.
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
+#include <cstring>
 #include <vector>
 
 #include "../../ir-multivector-retrieval_amd/csrc/kpp_rules.hpp"
@@ -55,6 +60,74 @@ static std::vector<double> other_order_prefix(const std::vector<float>& w) {
     base += tree[0];
   }
   return p;
+}
+
+// The wave's inclusive prefix sums (wave_inclusive_sum_f64 of kmeanspp.hpp).
+static void wave_inclusive(double* v) {
+  double o[64];
+  for (int k = 1; k <= 8; k <<= 1) {
+    memcpy(o, v, sizeof o);
+    for (int l = 0; l < 64; ++l)
+      if (l % 16 >= k) v[l] += o[l - k];
+  }
+  for (int l = 63; l >= 0; --l)
+    if (l / 16 % 2) v[l] += v[l / 16 * 16 - 1];
+  for (int l = 32; l < 64; ++l) v[l] += v[31];
+}
+
+// kpp_draw_wave<true> of kmeanspp.hpp from the draw r on: the decided row or
+// ~0.  With `subtract`, the exclusive sums are inclusive ones minus the own
+// value, the mistake that the check has to notice.
+static uint64_t wave_draw(const std::vector<float>& w, double r, bool subtract) {
+  const size_t n = w.size(), run_rows = 512, n_runs = (n + run_rows - 1) / run_rows;
+  const size_t per = (n_runs + 63) / 64;
+  std::vector<double> sums(64 * per, 0.0);
+  for (size_t q = 0; q < n_runs; ++q) {  // lane t of the run's wave adds rows t, t + 64, ...
+    double v[64] = {0};
+    for (size_t j = 0; j < run_rows / 64; ++j)
+      for (size_t t = 0; t < 64; ++t) {
+        const size_t i = q * run_rows + j * 64 + t;
+        if (i < n) v[t] += (double)w[i];
+      }
+    wave_inclusive(v);
+    sums[q] = v[63];
+  }
+  double share[64], incl[64];
+  for (size_t l = 0; l < 64; ++l) {
+    share[l] = 0.0;
+    for (size_t j = 0; j < per; ++j) share[l] += sums[l * per + j];
+  }
+  memcpy(incl, share, sizeof incl);
+  wave_inclusive(incl);
+  const double tot = incl[63], u = r * tot;
+  size_t fl = 0;
+  while (fl < 64 && !(fl * per < n_runs && u < incl[fl])) ++fl;
+  if (fl == 64) return ~0ull;
+  double before = subtract ? incl[fl] - share[fl] : fl ? incl[fl - 1] : 0.0;
+  const size_t f1 = std::min(n_runs, (fl + 1) * per);
+  size_t run = fl * per;
+  while (run + 1 < f1 && !(u < before + sums[run])) before += sums[run++];
+  double own[64], in[64];
+  for (size_t l = 0; l < 64; ++l) {
+    own[l] = 0.0;
+    for (size_t q = 0; q < 8; ++q) {
+      const size_t i = run * run_rows + l * 8 + q;
+      if (i < n) own[l] += (double)w[i];
+    }
+  }
+  memcpy(in, own, sizeof in);
+  wave_inclusive(in);
+  for (size_t l = 0; l < 64; ++l) {
+    double p = before + (subtract ? in[l] - own[l] : l ? in[l - 1] : 0.0);
+    for (size_t q = 0; q < 8; ++q) {
+      const size_t i = run * run_rows + l * 8 + q;
+      if (i >= n) return ~0ull;
+      const double prev = p;
+      p += (double)w[i];
+      if (u < p) return kpp_decides(r, tot, n, i, prev, p) ? i : ~0ull;
+    }
+  }
+  return ~0ull;
 }
 
 int main() {
@@ -135,6 +208,35 @@ int main() {
               (unsigned long long)decided, (unsigned long long)undecided, (unsigned long long)aimed,
               (unsigned long long)wrong);
   bad += (int)wrong;
+
+  // 3. the kernels' own sums, without and with the subtraction
+  uint64_t picks[2] = {0, 0}, off[2] = {0, 0};
+  for (int trial = 0; trial < 400; ++trial) {
+    const size_t n = 2 + next_u64() % 70000;
+    std::vector<float> w(n);
+    for (auto& x : w) x = (float)unit();
+    const size_t big = 1 + next_u64() % (n - 1);
+    w[big] = (float)std::pow(10.0, 6.0 + 10.0 * unit());
+    double total = 0.0;
+    for (float x : w) total += (double)x;
+    for (int d = 0; d < 50; ++d) {
+      // a draw that lands on one of the rows just before the large weight
+      const size_t back = std::min<size_t>(big, 1 + next_u64() % 1000), k = big - back;
+      double cum = 0.0;
+      for (size_t i = 0; i < k; ++i) cum += (double)w[i];
+      const double r = (cum + unit() * (double)w[k]) / total;
+      const uint64_t ref = reference_pick(w, r);
+      for (int sub = 0; sub < 2; ++sub) {
+        const uint64_t i = wave_draw(w, r, sub != 0);
+        picks[sub] += i != ~0ull;
+        off[sub] += i != ~0ull && i != ref;
+      }
+    }
+  }
+  std::printf("wave sums: %llu decided, %llu other rows; with the subtraction %llu and %llu\n",
+              (unsigned long long)picks[0], (unsigned long long)off[0],
+              (unsigned long long)picks[1], (unsigned long long)off[1]);
+  bad += off[0] != 0 || picks[0] < 1000 || off[1] == 0;
   std::printf("%s\n", bad ? "kpp rules check FAILED" : "kpp rules check passed");
   return bad ? 1 : 0;
 }
