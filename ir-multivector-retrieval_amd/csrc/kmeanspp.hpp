@@ -103,8 +103,7 @@ template <bool FUSED>
 __device__ __forceinline__ KppDraw kpp_draw_wave(const double* __restrict__ sums, uint32_t n_runs,
                                                  double share, const float* wm,
                                                  const float* patch, uint32_t patch_run,
-                                                 uint64_t n, uint64_t* prng,
-                                                 uint32_t exact_only) {
+                                                 uint64_t n, uint64_t* prng, bool leave_open) {
   const uint32_t lane = threadIdx.x % kWave;
   KppDraw out{kKppNone, kKppNone, 0, 0.0};
   const uint32_t per = (n_runs + kWave - 1) / kWave;
@@ -126,7 +125,7 @@ __device__ __forceinline__ KppDraw kpp_draw_wave(const double* __restrict__ sums
   out.r = kpp_float64(prng);
   const double u = out.r * tot;
   const uint64_t over = __ballot(q0 < n_runs && u < incl);
-  if (exact_only || !over) return out;  // u at or beyond the total: the tail rule decides
+  if (leave_open || !over) return out;  // u at or beyond the total: the tail rule decides
   const uint32_t fl = (uint32_t)__builtin_ctzll(over);
   // the run within that lane's share (its last when rounding leaves none)
   const uint32_t f0 = fl * per, f1 = f0 + per < n_runs ? f0 + per : n_runs;
@@ -224,7 +223,7 @@ __global__ __launch_bounds__(kKppThreads) void kpp_round_kernel(
     const float* __restrict__ xs, float* __restrict__ w, uint16_t* __restrict__ src,
     double* __restrict__ bsum, uint64_t bstride, float* __restrict__ patch,
     uint32_t* __restrict__ bad, const KppSeed* __restrict__ st_in, KppSeed* __restrict__ st_out,
-    float* __restrict__ cb, uint64_t n, uint32_t K, uint32_t NB, uint32_t exact_only) {
+    float* __restrict__ cb, uint64_t n, uint32_t K, uint32_t NB, uint32_t exact_every) {
   constexpr int DP = Pad<D>::value;
   constexpr float g = cand_gamma(D);
   constexpr uint32_t kPer = kKppRun / kWave;
@@ -271,7 +270,7 @@ __global__ __launch_bounds__(kKppThreads) void kpp_round_kernel(
       const bool non_finite = bad[m] < c;  // rng.zig:62
       KppDraw d = kpp_draw_wave<true>(bsum + bsel * bstride + (uint64_t)m * n_runs, n_runs, 0.0,
                                       wm, pm + patch_sel * kKppRun, S.patch_run, n, prng,
-                                      exact_only);
+                                      exact_every && (c + m) % exact_every == 0);
       if (non_finite) d.err = 9;  // NonFinite, before AllZero
       if (t == 0) s_draw = d;
     }
@@ -468,7 +467,7 @@ __device__ __forceinline__ void kpp_fallback_block(const float* __restrict__ wm,
 __global__ __launch_bounds__(kKppFallbackThreads) void kpp_draw_kernel(
     const float* __restrict__ w, const double* __restrict__ bsum, uint64_t bstride,
     const uint32_t* __restrict__ bad, KppSeed* __restrict__ st, uint64_t n, uint32_t K,
-    uint32_t n_runs, uint32_t exact_only, double* __restrict__ pre,
+    uint32_t n_runs, uint32_t exact_every, double* __restrict__ pre,
     FoldChunk* __restrict__ chunks, uint32_t nc) {
   constexpr uint32_t kPerShare = kKppFallbackThreads / kWave;  // lanes to a share of the runs
   __shared__ double shares[kWave];
@@ -492,7 +491,8 @@ __global__ __launch_bounds__(kKppFallbackThreads) void kpp_draw_kernel(
     for (int q = 0; q < 4; ++q) prng[q] = in.s[q];
     const bool non_finite = bad[m] < in.next;  // rng.zig:62
     const KppDraw d = kpp_draw_wave<false>(sums, n_runs, shares[t], w + (uint64_t)m * n, nullptr,
-                                           kKppNone, n, prng, exact_only);
+                                           kKppNone, n, prng,
+                                           exact_every && (in.next + m) % exact_every == 0);
     if (t == 0) {
       KppSeed& o = st[m];
       const int32_t err = non_finite ? 9 : d.err;  // NonFinite before AllZero

@@ -973,11 +973,11 @@ struct Launch {
   static void kpp_round(const float *xs, float *w, uint16_t *src, double *bsum,
                         uint64_t bstride, float *patch, uint32_t *bad, const KppSeed *in,
                         KppSeed *out, float *cb, uint64_t n, uint32_t M, uint32_t K, uint32_t NB,
-                        uint32_t exact_only, hipStream_t s) {
+                        uint32_t exact_every, hipStream_t s) {
     auto *kernel = NB * kKppRuns <= kKppFusedRuns ? kpp_round_kernel<D, true>
                                                   : kpp_round_kernel<D, false>;
     kernel<<<dim3(NB, M), kKppThreads, 0, s>>>(xs, w, src, bsum, bstride, patch, bad, in, out, cb,
-                                               n, K, NB, exact_only);
+                                               n, K, NB, exact_every);
   }
   static void fold(const float *sorted, const uint32_t *counts, const uint32_t *start,
                    float *cb, const uint32_t *done, const uint32_t *order, uint64_t n, uint32_t M,
@@ -1108,10 +1108,11 @@ int kmeanspp(DeviceState &ds, hipStream_t s, const SubspaceGroup *groups, uint32
     return st;
   double *fold_pre = as<double>(ds.fold_pre);
   FoldChunk *fold_chunks = as<FoldChunk>(ds.fold_chunks);
-  // TAC_GPU_KPP_EXACT=1: every draw takes the exact sequential evaluation
-  // (the same picks, slower; the parallel band test is skipped).
+  // TAC_GPU_KPP_EXACT=v: the draws of codeword c in the group's subspace m with
+  // (c + m) % v == 0 take the exact sequential evaluation (v = 1: every draw;
+  // the same picks, slower; the parallel band test is skipped).
   const char *exact_env = getenv("TAC_GPU_KPP_EXACT");
-  const uint32_t exact_only = exact_env != nullptr && exact_env[0] == '1';
+  const uint32_t exact_every = exact_env != nullptr ? (uint32_t)std::max(0, atoi(exact_env)) : 0u;
   KppSeed *state[2] = {as<KppSeed>(ds.kpp_state), as<KppSeed>(ds.kpp_state) + M};
   float *w = as<float>(ds.kpp_w);
   float *patch = as<float>(ds.kpp_patch);
@@ -1134,7 +1135,7 @@ int kmeanspp(DeviceState &ds, hipStream_t s, const SubspaceGroup *groups, uint32
         if (!fused && launch > 0) {
           kpp_draw_kernel<<<g.Mh, kKppFallbackThreads, 0, g.s>>>(
               w + m0 * n, bsum + m0 * n_runs, (uint64_t)M * n_runs, bad + m0,
-              state[launch & 1] + m0, n, K, n_runs, exact_only, fold_pre + m0 * nfc,
+              state[launch & 1] + m0, n, K, n_runs, exact_every, fold_pre + m0 * nfc,
               fold_chunks + m0 * nfc, nfc);
           LAUNCH_TRY("kpp_draw_kernel");
         }
@@ -1142,7 +1143,7 @@ int kmeanspp(DeviceState &ds, hipStream_t s, const SubspaceGroup *groups, uint32
                                 bsum + m0 * n_runs, (uint64_t)M * n_runs,
                                 patch + m0 * 2 * kKppRun, bad + m0, state[launch & 1] + m0,
                                 state[~launch & 1] + m0, cb + m0 * K * D, n, g.Mh, K, NB,
-                                exact_only, g.s));
+                                exact_every, g.s));
         LAUNCH_TRY("kpp_round_kernel");
       }
       // Pending draws are made every 32 rounds (an idle launch takes 3 us): a
@@ -1170,7 +1171,7 @@ int kmeanspp(DeviceState &ds, hipStream_t s, const SubspaceGroup *groups, uint32
   std::vector<KppSeed> hs(M);
   st = init();
   for (uint32_t left = K; left > 0;) {
-    if (!st) st = rounds(exact_only && fused ? std::min(left, 2u) : left);
+    if (!st) st = rounds(exact_every == 1 && fused ? std::min(left, 2u) : left);
     // The call's stream waits for the other groups, also after an error.
     for (uint32_t h = 1; h < H; ++h) {
       HIP_TRY(hipEventRecord(ds.aux_join[h - 1], groups[h].s));

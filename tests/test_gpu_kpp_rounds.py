@@ -34,6 +34,22 @@ def test_seeds_match_oracle(gpu, monkeypatch, n, m, dsub, ksub, exact):
     assert np.array_equal(got.codebooks.view(np.uint32), ref.codebooks.reshape(-1).view(np.uint32))
 
 
+@pytest.mark.parametrize("n,m,dsub,ksub", [(5000, 8, 4, 100), (513, 3, 2, 150), (100_001, 5, 8, 70),
+                                           (270_001, 3, 4, 40)])
+@pytest.mark.parametrize("every", [2, 3, 7, 40])
+def test_open_draws_between_decided_ones(gpu, monkeypatch, n, m, dsub, ksub, every):
+    """Only some draws of some subspaces are left open: the drawn run's weights
+    go back from the patch, the exact draw resumes the subspace, and it catches
+    up while the others pass by (every 32 rounds, and at the end).  The 513 rows
+    hold some 221 distinct ones: more seeds than that would be AllZero."""
+    x = _rows(n, m * dsub, n + every, distinct=n // 2 if n % 2 else None)
+    monkeypatch.setenv("TAC_GPU_KPP_EXACT", str(every))
+    got = pq.train(x, m * dsub, 77, m=m, ksub=ksub, max_iters=1, tol=NEVER)
+    ref = orc.pq_train(x, m * dsub, m, ksub, seed=77, max_iters=1, tol=NEVER, n_threads=16)
+    assert ref.status == 0
+    assert np.array_equal(got.codebooks.view(np.uint32), ref.codebooks.reshape(-1).view(np.uint32))
+
+
 @pytest.mark.parametrize("n", [3000, 270_000])
 def test_errors_of_the_lowest_subspace(gpu, n):
     """All weights zero after the first pick, and distances that overflow."""
