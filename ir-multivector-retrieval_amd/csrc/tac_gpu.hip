@@ -26,6 +26,7 @@
 #include "query_kernels.hpp"
 #include "tac_kernels.hpp"
 #include "tac_phases.hpp"
+#include "download.hpp"
 
 #include <hip/hip_runtime.h>
 
@@ -43,7 +44,6 @@
 #include <condition_variable>
 #include <mutex>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -117,7 +117,6 @@ struct DeviceState {
   hipEvent_t stage_ev[kStageBufs] = {};
   bool stage_pending[kStageBufs] = {};
   // pinned buffers of large downloads (download_host)
-  static constexpr int kDownBufs = 4;
   void *down = nullptr;
   hipEvent_t down_ev[kDownBufs] = {};
   // words of pinned host memory that kernels write results to (host_words)
@@ -258,91 +257,60 @@ int upload_host(DeviceState &ds, void *dst, const void *src, size_t bytes, hipSt
   return TAC_OK;
 }
 
-constexpr size_t kDownChunk = 4u << 20;  // most bytes per staged copy back
-constexpr size_t kDownMin = 2u << 20;    // smaller outputs copy to pageable memory directly
+// The port of download() over one call's stream.  `flag` is a host word that the
+// kernels before the copy may raise, or null.
+struct HipDownload {
+  DeviceState &ds;
+  const char *src;
+  hipStream_t s;
+  const uint32_t *flag;
+  int dev = 0;
 
-// Device-to-host copy of `bytes` into pageable memory, ordered behind the work
-// on s; returns when dst is written.  Large copies pass in chunks through a
-// ring of pinned buffers: kStageThreads host threads each write their share of
-// every chunk to dst (and take its page faults, when dst is fresh memory)
-// while the DMA fetches the next ones.  A chunk costs some 15 us beside its
-// bytes, so there are at least four of at most 4 MB.  Decode of 65,537 rows
-// to 16.8 MB: 620 us a call, 715 with chunks of 1 MB, 1,040 with a
-// hipMemcpyAsync to the same pageable memory, which one thread empties.  With
-// skip, a host word that the kernels before the copy may raise, dst is left
-// alone when it is raised.
+  bool ring() {
+    if (!ds.down && hipHostMalloc(&ds.down, kDownBufs * kDownChunk, hipHostMallocDefault) !=
+                        hipSuccess) {
+      ds.down = nullptr;
+      (void)hipGetLastError();  // not the next launch's
+      return false;
+    }
+    for (hipEvent_t &e : ds.down_ev)
+      if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+        e = nullptr;
+        (void)hipGetLastError();
+        return false;
+      }
+    return hipGetDevice(&dev) == hipSuccess;
+  }
+  const char *buffer(size_t b) const { return static_cast<char *>(ds.down) + b * kDownChunk; }
+  int fetch(size_t b, size_t off, size_t len) {
+    const hipError_t e = hipMemcpyAsync(static_cast<char *>(ds.down) + b * kDownChunk, src + off,
+                                        len, hipMemcpyDeviceToHost, s);
+    return (int)(e != hipSuccess ? e : hipEventRecord(ds.down_ev[b], s));
+  }
+  int wait(size_t b) { return (int)hipEventSynchronize(ds.down_ev[b]); }
+  int attach() { return (int)hipSetDevice(dev); }
+  bool skip() const { return flag && __atomic_load_n(flag, __ATOMIC_ACQUIRE); }
+  int drain() { return (int)hipStreamSynchronize(s); }
+  int direct(void *dst, size_t bytes) {
+    hipError_t e = hipSuccess;
+    if (flag && ((e = hipStreamSynchronize(s)) != hipSuccess || skip())) return (int)e;
+    e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
+    return (int)(e != hipSuccess ? e : hipStreamSynchronize(s));
+  }
+  template <class F>
+  std::thread spawn(F f) {
+    return std::thread(f);
+  }
+};
+
+// Device-to-host copy of `bytes`, ordered behind the work on s; returns when
+// dst is written.  With skip, dst is left alone when that word is raised.
 int download_host(DeviceState &ds, void *dst, const void *src, size_t bytes, hipStream_t s,
                   const uint32_t *skip = nullptr) {
   if (bytes == 0) return TAC_OK;
-  if (bytes < kDownMin) {
-    if (skip) {
-      HIP_TRY(hipStreamSynchronize(s));
-      if (__atomic_load_n(skip, __ATOMIC_ACQUIRE)) return TAC_OK;
-    }
-    HIP_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
-    return TAC_OK;
-  }
-  constexpr int T = DeviceState::kStageThreads, B = DeviceState::kDownBufs;
-  if (!ds.down) HIP_TRY(hipHostMalloc(&ds.down, B * kDownChunk, hipHostMallocDefault));
-  for (int b = 0; b < B; ++b)
-    if (!ds.down_ev[b]) HIP_TRY(hipEventCreateWithFlags(&ds.down_ev[b], hipEventDisableTiming));
-  const size_t chunk = std::min(kDownChunk, (bytes / B + 65535) / 65536 * 65536);
-  const size_t nch = (bytes + chunk - 1) / chunk;
-  int dev = 0;
-  HIP_TRY(hipGetDevice(&dev));
-  auto fetch = [&](size_t c) -> hipError_t {  // chunk c into buffer c % B
-    const size_t b = c % B, off = c * chunk;
-    const hipError_t e = hipMemcpyAsync(static_cast<char *>(ds.down) + b * kDownChunk,
-                                        static_cast<const char *>(src) + off,
-                                        std::min(bytes - off, chunk), hipMemcpyDeviceToHost, s);
-    return e != hipSuccess ? e : hipEventRecord(ds.down_ev[b], s);
-  };
-  const size_t ahead = std::min<size_t>(nch, B);
-  for (size_t c = 0; c < ahead; ++c) HIP_TRY(fetch(c));
-  std::atomic<size_t> issued{ahead};            // chunks whose event is recorded
-  std::atomic<int> left[DeviceState::kDownBufs];  // threads yet to empty a buffer
-  for (auto &l : left) l = T;
-  std::atomic<int> failed{(int)hipSuccess};
-  auto work = [&](int tid) {
-    hipError_t e = hipSetDevice(dev);
-    for (size_t c = 0; c < nch && e == hipSuccess; ++c) {
-      while (issued.load(std::memory_order_acquire) <= c) {
-        if (failed.load(std::memory_order_acquire) != (int)hipSuccess) return;
-        std::this_thread::yield();
-      }
-      if ((e = hipEventSynchronize(ds.down_ev[c % B])) != hipSuccess) break;
-      if (skip && __atomic_load_n(skip, __ATOMIC_ACQUIRE)) return;
-      const size_t off = c * chunk, len = std::min(bytes - off, chunk);
-      // shares of whole pages
-      const size_t share = (len / T + 4095) / 4096 * 4096;
-      const size_t lo = std::min(len, share * tid);
-      const size_t hi = tid + 1 == T ? len : std::min(len, lo + share);
-      memcpy(static_cast<char *>(dst) + off + lo,
-             static_cast<char *>(ds.down) + c % B * kDownChunk + lo, hi - lo);
-      if (left[c % B].fetch_sub(1, std::memory_order_acq_rel) == 1 && c + B < nch) {
-        // the last to leave the buffer refills it; buffers empty in order
-        left[c % B].store(T, std::memory_order_release);
-        if ((e = fetch(c + B)) == hipSuccess) issued.fetch_add(1, std::memory_order_acq_rel);
-      }
-    }
-    if (e != hipSuccess) failed.store((int)e, std::memory_order_release);
-  };
-  std::vector<std::thread> helpers;
-  helpers.reserve(T);
-  int st = TAC_OK;
-  try {
-    for (int t = 1; t < T; ++t) helpers.emplace_back(work, t);
-  } catch (const std::system_error &) {
-    // no thread to be had: the copy fails as the other allocations do
-    failed.store((int)hipErrorOutOfMemory, std::memory_order_release);
-  }
-  if (failed.load(std::memory_order_acquire) == (int)hipSuccess) work(0);
-  for (auto &h : helpers) h.join();
-  const hipError_t drained = hipStreamSynchronize(s);  // no copy outlives the call
-  if (failed.load() != (int)hipSuccess) st = hip_status("download", (hipError_t)failed.load());
-  if (!st && drained != hipSuccess) st = hip_status("hipStreamSynchronize", drained);
-  return st;
+  HipDownload port{ds, static_cast<const char *>(src), s, skip};
+  const int e = download(port, dst, bytes);
+  return e ? hip_status("download", (hipError_t)e) : TAC_OK;
 }
 
 // Order this call after the previous one that used the workspace.
