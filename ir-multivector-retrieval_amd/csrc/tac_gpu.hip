@@ -266,6 +266,16 @@ struct HipDownload {
   const uint32_t *flag;
   int dev = 0;
 
+  // Memory that the runtime knows (pinned, managed, a device's): the DMA writes
+  // it itself.
+  bool known(const void *dst) const {
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, dst) != hipSuccess) {
+      (void)hipGetLastError();  // pageable memory is an invalid value to some runtimes
+      return false;
+    }
+    return a.type != hipMemoryTypeUnregistered;
+  }
   bool ring() {
     if (!ds.down && hipHostMalloc(&ds.down, kDownBufs * kDownChunk, hipHostMallocDefault) !=
                         hipSuccess) {

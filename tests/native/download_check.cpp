@@ -1,6 +1,6 @@
 // CPU check of the staged device-to-host copy (csrc/download.hpp): every size at
 // the edges of its chunks, with a thread that cannot be made (each of the
-// seven), no ring, a fetch that fails and a raised skip word.  The device is a
+// seven), no ring, a pinned output, a fetch that fails and a raised skip word.  The device is a
 // buffer in memory whose fetches run at once.
 #include <cstdio>
 #include <new>
@@ -16,11 +16,12 @@ struct Port {
   std::vector<char> mem = std::vector<char>(kDownBufs * kDownChunk);
   int spawn_limit = kDownThreads;  // threads that can be made
   bool no_memory = false;          // the one past them: bad_alloc, else system_error
-  bool have_ring = true, raised = false;
+  bool have_ring = true, pinned = false, raised = false;
   size_t fail_at = ~(size_t)0;  // offset whose fetch fails
   int directs = 0, made = 0;
   std::atomic<size_t> fetched{0};
 
+  bool known(const void *) const { return pinned; }
   bool ring() { return have_ring; }
   const char *buffer(size_t b) const { return mem.data() + b * kDownChunk; }
   int fetch(size_t b, size_t off, size_t len) {
@@ -80,6 +81,11 @@ int main() {
     Port none{src};
     none.have_ring = false;
     expect(download(none, dst.data(), bytes) == 0 && dst == src && none.made == 0, "no ring", bytes, 0);
+    Port pinned{src};
+    pinned.pinned = true;
+    std::fill(dst.begin(), dst.end(), 1);
+    expect(download(pinned, dst.data(), bytes) == 0 && dst == src, "pinned", bytes, 0);
+    expect(pinned.directs == 1 && pinned.made == 0, "pinned copies", bytes, 0);
     for (size_t c = 0; staged && c < 9; ++c) {
       const size_t chunk = std::min(kDownChunk, (bytes / kDownBufs + 65535) / 65536 * 65536);
       if (c * chunk >= bytes) break;
