@@ -28,7 +28,10 @@ namespace tacgpu {
 constexpr int kDownThreads = 8;
 constexpr int kDownBufs = 4;
 constexpr size_t kDownChunk = 4u << 20;  // most bytes per staged copy
-constexpr size_t kDownMin = 2u << 20;    // smaller outputs take the direct copy
+// Smaller outputs take the direct copy.  Decode, us a call, direct | staged: 2 MB
+// 169 | 243, 3 MB 227 | 262, 4 MB 288 | 291, 5 MB 350 | 303-329, 6 MB 410 | 330,
+// 8 MB 540 | 397.
+constexpr size_t kDownMin = 5u << 20;
 
 // Copies `bytes` to dst; returns when dst is written.  Large copies to pageable
 // memory pass in chunks through the ring: kDownThreads host threads each write

@@ -59,7 +59,8 @@ static void expect(bool ok, const char *what, size_t bytes, int arg) {
 }
 
 int main() {
-  const size_t sizes[] = {1, kDownMin - 1, kDownMin, kDownMin + 1, 3 * kDownMin + 4097,
+  const size_t sizes[] = {1, kDownMin - 1, kDownMin, kDownMin + 1, kDownMin + 70000,
+                          3 * kDownMin + 4097,
                           4 * kDownChunk, 4 * kDownChunk + 1, 9 * kDownChunk + 65537};
   for (size_t bytes : sizes) {
     std::vector<char> src(bytes);

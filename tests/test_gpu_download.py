@@ -1,4 +1,4 @@
-"""Host outputs at the edges of the staged download (2 MB, its chunks of at most
+"""Host outputs at the edges of the staged download (5 MB, its chunks of at most
 4 MB, its ring of four): decode round trips, and a bad code leaves `out` alone."""
 import ctypes
 
@@ -11,7 +11,8 @@ from tac_gpu import errors, lib, pq
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("floats", [1, 524_287, 524_288, 524_289, 4_194_304, 4_194_305, 9_000_001])
+@pytest.mark.parametrize("floats", [1, 524_287, 524_288, 524_289, 1_310_719, 1_310_720,
+                                    1_310_721, 4_194_304, 4_194_305, 9_000_001])
 def test_decode_sizes(gpu, floats):
     rng = np.random.default_rng(floats)
     cb = rng.standard_normal(256).astype(np.float32)
@@ -21,8 +22,8 @@ def test_decode_sizes(gpu, floats):
         assert np.array_equal(p.decode_many(codes), cb[codes])
 
 
-def test_bad_code_leaves_the_output(gpu):
-    n = 1_000_000
+@pytest.mark.parametrize("n", [1_000_000, 2_000_000])
+def test_bad_code_leaves_the_output(gpu, n):
     codes = np.zeros((n, 1), np.uint8)
     codes[-1] = 9
     out = np.full(n, 7.0, np.float32)
@@ -37,7 +38,7 @@ def test_bad_code_leaves_the_output(gpu):
     assert call() == 0 and (out == 0.0).all()
 
 
-@pytest.mark.parametrize("floats", [524_287, 4_194_305, 9_000_001])
+@pytest.mark.parametrize("floats", [524_287, 1_310_721, 4_194_305, 9_000_001])
 def test_pinned_output(gpu, floats):
     rng = np.random.default_rng(floats)
     cb = rng.standard_normal(256).astype(np.float32)
