@@ -98,7 +98,7 @@ struct DeviceState {
   hipEvent_t last_done = nullptr;
   // training / encode workspace
   Buffer xs, codes, e, hist, counts, start, sorted, flags, scal, trace, io_in, io_out, io_cb,
-      io_init, counter, kpp_state, kpp_w, kpp_bsum, kpp_bad, status, io_aux, io_out2, scan_sums,
+      io_init, counter, kpp_state, kpp_w, kpp_bsum, kpp_bad, io_aux, io_out2, scan_sums,
       io_x1, io_x2, io_x3, crc_tables, doc_state, doc_slices, fold_pre, fold_chunks, cand_nbr, cand_defer, cand_count, cand_anchor, cand_grid, kpp_src, kpp_patch,
       fold_order, cell_par, cell_cids, cell_ccnt, cell_rec, cell_list;
   // token-aware clustering
@@ -1922,7 +1922,7 @@ int tac_gpu_release_workspace(void) {
   Buffer *bufs[] = {&ds->xs,        &ds->codes,   &ds->e,         &ds->hist,     &ds->counts,
                     &ds->start,     &ds->sorted,  &ds->flags,     &ds->scal,     &ds->trace,
                     &ds->io_in,     &ds->io_out,  &ds->io_cb,     &ds->io_init,  &ds->counter,
-                    &ds->kpp_state, &ds->kpp_w,   &ds->kpp_bsum,  &ds->kpp_bad,  &ds->status,
+                    &ds->kpp_state, &ds->kpp_w,   &ds->kpp_bsum,  &ds->kpp_bad,
                     &ds->io_aux,    &ds->io_out2, &ds->scan_sums, &ds->io_x1,    &ds->io_x2,
                     &ds->io_x3,     &ds->crc_tables, &ds->doc_state, &ds->doc_slices, &ds->fold_pre,  &ds->fold_chunks,
                     &ds->tac_v,     &ds->tac_idx, &ds->tac_offs,  &ds->tac_G,
