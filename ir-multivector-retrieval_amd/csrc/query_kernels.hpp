@@ -73,17 +73,18 @@ __device__ __forceinline__ uint32_t load_u32_le(const uint8_t* p) {
   return (uint32_t)p[0] | (uint32_t)p[1] << 8 | (uint32_t)p[2] << 16 | (uint32_t)p[3] << 24;
 }
 
-// One block of W waves per candidate document (grid-stride over candidates).
-// A wave covers QP = n_q rounded up to a power of two (at most 64) query
-// tokens and S = 64 / QP slots; lane (s, i) takes query token i0 + i against
-// R document tokens of slot s at a time, for every token k
+// A team of one block of W waves, or with WAVES of one of its waves, per
+// candidate document (the host chooses by the documents' mean length),
+// grid-stride over candidates.  A wave covers QP = n_q rounded up to a power of
+// two (at most 64) query tokens and S = 64 / QP slots; lane (s, i) takes query
+// token i0 + i against R document tokens of slot s at a time, for every token k
 //   cent  = dot(q_i, centroid[c_k])            (centroid rows staged in LDS)
 //   res   = sum over m of table[m][code_km][i]  (in m order, from 0)
 //   score = cent + norm_k * res
 // and keeps the first k of its running maximum (strict >, from -inf).  The
 // slots and waves of a query token then merge (larger value; on equal values
 // the earlier k, which keeps the sign of a zero maximum the reference would
-// keep), and wave 0 folds best_0 + best_1 + ... in i order (0 for an empty
+// keep), and the team's wave 0 folds best_0 + best_1 + ... in i order (0 for an empty
 // document).  Layout checks follow refine.zig:51-65,107-114; a failing
 // candidate scores 0, `first_bad` keeps the lowest one with its status
 // (candidate << 32 | status) and `any_bad`, a word of pinned host memory,
@@ -99,6 +100,7 @@ __device__ __forceinline__ uint32_t load_u32_le(const uint8_t* p) {
 // flight while the dots run: 31 us and 8 us.  Four tokens a lane spill
 // registers (73 against 51 us a call at 32 x 1,000).
 constexpr uint32_t kRefineTileFloats = 8192;  // most row floats, and codes, of a tile
+constexpr uint32_t kRefineWaveFloats = 1536;  // of a tile that one wave works on
 
 __host__ __device__ inline uint32_t refine_qp(uint32_t n_q) {
   uint32_t qp = 1;
@@ -112,20 +114,22 @@ __host__ __device__ inline uint32_t refine_stride(uint32_t dim, bool fast) {
   return fast ? dim + 4 : dim + 1;
 }
 
-// Tokens of a tile: at most 8,192 row floats and 8,192 codes.
-inline uint32_t refine_tile(uint32_t dim, uint32_t M, uint32_t most) {
-  const uint32_t w = dim > M ? dim : M, t = kRefineTileFloats / w;
+// Tokens of a tile: at most `floats` row floats and as many codes, or one.
+inline uint32_t refine_tile(uint32_t dim, uint32_t M, uint32_t floats, uint32_t most) {
+  const uint32_t w = dim > M ? dim : M, t = floats / w;
   return t > most ? most : (t ? t : 1u);
 }
 
-// Dynamic LDS floats of a block of `waves` waves: the queries, the tile's
+// Dynamic LDS floats of the queries, and of a team of `waves` waves: its tile's
 // centroid rows, per wave 64 best values and their token indices, and the
 // tile's codes as u16, in rows of whole 16 bytes.
-inline uint64_t refine_lds_floats(uint32_t n_q, uint32_t dim, bool fast, uint32_t waves,
-                                  uint32_t M, uint64_t tile) {
-  const uint32_t ld = refine_stride(dim, fast);
-  return ((n_q + tile) * ld + 3) / 4 * 4 + waves * 128 +
-         (M <= kRefineTileFloats ? tile * ((M + 7ull) / 8 * 4) : 0ull);
+__host__ __device__ inline uint32_t refine_query_floats(uint32_t n_q, uint32_t ld) {
+  return (n_q * ld + 3) / 4 * 4;
+}
+__host__ __device__ inline uint32_t refine_team_floats(uint32_t ld, uint32_t waves, uint32_t M,
+                                                       uint32_t tile) {
+  return (tile * ld + 3) / 4 * 4 + waves * 128 +
+         (M <= kRefineTileFloats ? tile * ((M + 7) / 8 * 4) : 0u);
 }
 
 // dot(q_i, centroid row) of R rows in LDS; FAST is vec.dot's 4-lane form.
@@ -239,21 +243,35 @@ __device__ __forceinline__ void refine_keep(float& b, uint32_t& bk, float o, uin
 }
 
 // FAST: dims 64 and 128 (vec.dot's 4-lane form), with 16-byte aligned
-// centroid and query arrays; else R is 1 and ref_dot serves any dim.
-template <int R, bool FAST>
+// centroid and query arrays; else R is 1 and ref_dot serves any dim.  WAVES: a
+// candidate to each wave instead of each block, with the queries shared.
+template <int R, bool FAST, bool WAVES>
 __global__ __launch_bounds__(512, 4) void refine_kernel(
     RefineIndex ix, const float* __restrict__ q, uint32_t n_q, const float* __restrict__ table,
     const uint32_t* __restrict__ doc_ids, uint32_t n_cand, uint32_t TT, float* __restrict__ scores,
     unsigned long long* __restrict__ first_bad, uint32_t* __restrict__ any_bad) {
   static_assert(FAST || R == 1, "the generic dot takes one token at a time");
   extern __shared__ __attribute__((aligned(16))) float lds[];
-  const uint32_t w = threadIdx.x / 64, lane = threadIdx.x % 64, W = blockDim.x / 64;
+  const uint32_t lane = threadIdx.x % 64;
+  // The team: W waves, this one its wave w, this thread its thread tid of nt.
+  const uint32_t teams = WAVES ? blockDim.x / 64 : 1, team = WAVES ? threadIdx.x / 64 : 0;
+  const uint32_t W = WAVES ? 1 : blockDim.x / 64, w = WAVES ? 0 : threadIdx.x / 64;
+  const uint32_t tid = WAVES ? lane : threadIdx.x, nt = WAVES ? 64 : blockDim.x;
+  auto team_any = [](bool v) -> bool {  // and the team's LDS accesses ordered
+    if constexpr (WAVES) {
+      wave_lds_sync();
+      return __any(v);
+    } else {
+      return __syncthreads_or(v);
+    }
+  };
   const uint32_t ld = refine_stride(ix.dim, FAST);
   const uint32_t QP = refine_qp(n_q), S = 64 / QP;
   const uint32_t slot = lane / QP, qi = lane % QP;
-  float* qs = lds;                         // [n_q][ld]
-  float* rows = lds + (size_t)n_q * ld;    // [TT][ld]
-  float* bestv = lds + ((n_q + TT) * ld + 3) / 4 * 4;               // [W][64]
+  float* qs = lds;  // [n_q][ld]
+  float* rows = lds + refine_query_floats(n_q, ld) +
+                team * refine_team_floats(ld, W, ix.M, TT);         // [TT][ld]
+  float* bestv = rows + (TT * ld + 3) / 4 * 4;                      // [W][64]
   uint32_t* bestk = reinterpret_cast<uint32_t*>(bestv + 64 * W);    // [W][64]
   uint16_t* scodes = reinterpret_cast<uint16_t*>(bestk + 64 * W);   // [TT][lc]
   const bool long_codes = ix.M > kRefineTileFloats;
@@ -267,8 +285,9 @@ __global__ __launch_bounds__(512, 4) void refine_kernel(
     for (uint32_t f = threadIdx.x; f < n_q * ix.dim; f += blockDim.x)
       qs[(f / ix.dim) * ld + f % ix.dim] = q[f];
   }
+  if constexpr (WAVES) __syncthreads();  // the teams' only common point
   const uint32_t cb = ix.K <= 256 ? 1u : 2u, step = ix.K * n_q;
-  for (uint32_t cand = blockIdx.x; cand < n_cand; cand += gridDim.x) {
+  for (uint32_t cand = blockIdx.x * teams + team; cand < n_cand; cand += gridDim.x * teams) {
     const uint64_t doc = doc_ids[cand];
     uint32_t st = kRefineOk;
     uint32_t n_d = 0;
@@ -315,7 +334,7 @@ __global__ __launch_bounds__(512, 4) void refine_kernel(
         if (long_codes) {
         } else if (words) {
           const uint32_t* src = reinterpret_cast<const uint32_t*>(codes0 + (uint64_t)k0 * ix.M);
-          for (uint32_t f = threadIdx.x; f < cnt * ix.M / 4; f += blockDim.x) {
+          for (uint32_t f = tid; f < cnt * ix.M / 4; f += nt) {
             const uint32_t v = src[f];
             const uint32_t c0 = v & 0xFFu, c1 = (v >> 8) & 0xFFu, c2 = (v >> 16) & 0xFFu,
                            c3 = v >> 24;
@@ -324,7 +343,7 @@ __global__ __launch_bounds__(512, 4) void refine_kernel(
           }
         } else {
           const uint8_t* src = codes0 + (uint64_t)k0 * ix.M * cb;
-          for (uint32_t f = threadIdx.x; f < cnt * lc; f += blockDim.x) {
+          for (uint32_t f = tid; f < cnt * lc; f += nt) {
             const uint32_t mm = f % lc;
             const uint8_t* p = src + ((uint64_t)(f / lc) * ix.M + mm) * cb;
             uint32_t c = 0;
@@ -335,7 +354,7 @@ __global__ __launch_bounds__(512, 4) void refine_kernel(
         }
         // centroid rows of tokens k0 .. k0 + cnt - 1
         const uint32_t units = FAST ? ix.dim / 4 : ix.dim;
-        for (uint32_t f = threadIdx.x; f < cnt * units; f += blockDim.x) {
+        for (uint32_t f = tid; f < cnt * units; f += nt) {
           const uint32_t s = f / units, d = f % units;
           const uint8_t* idp = ids + 4ull * (k0 + s);
           const uint32_t cid =
@@ -349,7 +368,7 @@ __global__ __launch_bounds__(512, 4) void refine_kernel(
             rows[s * ld + d] = ix.centroids[(uint64_t)cid * ix.dim + d];
           }
         }
-        if (__syncthreads_or(bad)) {  // also: the rows (and the queries) are staged
+        if (team_any(bad)) {  // also: the rows (and the queries) are staged
           st = kRefineLayoutCorrupt;
           break;
         }
@@ -383,7 +402,7 @@ __global__ __launch_bounds__(512, 4) void refine_kernel(
               bk = k0 + t[r];
             }
         }
-        if (__syncthreads_or(bad)) {  // also: the rows may be overwritten
+        if (team_any(bad)) {  // also: the rows may be overwritten
           st = kRefineLayoutCorrupt;
           break;
         }
@@ -394,9 +413,11 @@ __global__ __launch_bounds__(512, 4) void refine_kernel(
         const uint32_t ok = __shfl_xor(bk, off, 64);
         refine_keep(b, bk, o, ok);
       }
-      bestv[threadIdx.x] = b;
-      bestk[threadIdx.x] = bk;
-      __syncthreads();
+      if constexpr (!WAVES) {
+        bestv[threadIdx.x] = b;
+        bestk[threadIdx.x] = bk;
+        __syncthreads();
+      }
       if (w == 0) {
         for (uint32_t ww = 1; ww < W; ++ww)
           refine_keep(b, bk, bestv[ww * 64 + lane], bestk[ww * 64 + lane]);
@@ -405,9 +426,9 @@ __global__ __launch_bounds__(512, 4) void refine_kernel(
           total = total + __uint_as_float(
                               (uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(b), (int)j));
       }
-      __syncthreads();  // wave 0 has read the best values
+      if constexpr (!WAVES) __syncthreads();  // wave 0 has read the best values
     }
-    if (threadIdx.x == 0) {
+    if (tid == 0) {
       scores[cand] = st == kRefineOk ? total : 0.0f;
       if (st != kRefineOk) {
         atomicMin(first_bad, (unsigned long long)cand << 32 | st);

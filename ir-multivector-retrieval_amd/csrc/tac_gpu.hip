@@ -2563,27 +2563,35 @@ int validate_refine(const tac_doc_index *ix, uint64_t table_len, uint32_t n_q) {
   return refine_fits(n_q, ix->dim);
 }
 
-// Up to 512 candidates, or rows past 64 floats: 8 waves a block and tiles of
-// 128 tokens, so that a document is one or two steps long; more candidates
-// fill the chip by themselves and take 4 waves and tiles of 64, whose LDS
-// lets 5 blocks share a CU.  Call times in us (8 waves x 128 | 4 x 64; 32
-// query tokens, m16, documents of 1-100 tokens): dim 64 at 250 candidates
-// 36.2 | 42.7, 500 39.0 | 44.6, 1,000 53.6 | 48.9, 4,000 130 | 106; dim 128
-// at 1,000 67.9 | 78.3, 4,000 169 | 207.
-template <int R, bool FAST>
+template <int R, bool FAST, bool WAVES>
 int refine_launch(const RefineIndex &r, const float *d_q, uint32_t n_q, const float *d_table,
-                  const uint32_t *d_ids, uint32_t n_cand, float *d_scores,
-                  unsigned long long *first_bad, uint32_t *any_bad, hipStream_t s) {
-  const bool wide = n_cand <= 512 || r.dim > 64;
-  const uint32_t waves = wide ? 8 : 4, tile = refine_tile(r.dim, r.M, wide ? 128 : 64);
-  const uint32_t lds =
-      (uint32_t)(refine_lds_floats(n_q, r.dim, FAST, waves, r.M, tile) * sizeof(float));
-  if (int st = raise_lds((const void *)refine_kernel<R, FAST>, lds, 0)) return st;
-  const unsigned blocks = n_cand < 16384 ? n_cand : 16384;
-  refine_kernel<R, FAST><<<blocks, 64 * waves, lds, s>>>(r, d_q, n_q, d_table, d_ids, n_cand,
-                                                         tile, d_scores, first_bad, any_bad);
+                  const uint32_t *d_ids, uint32_t n_cand, uint32_t waves, uint32_t tile,
+                  uint32_t lds, float *d_scores, unsigned long long *first_bad,
+                  uint32_t *any_bad, hipStream_t s) {
+  if (int st = raise_lds((const void *)refine_kernel<R, FAST, WAVES>, lds, 0)) return st;
+  const uint32_t want = WAVES ? (n_cand + waves - 1) / waves : n_cand;
+  refine_kernel<R, FAST, WAVES><<<std::min(want, 16384u), 64 * waves, lds, s>>>(
+      r, d_q, n_q, d_table, d_ids, n_cand, tile, d_scores, first_bad, any_bad);
   LAUNCH_TRY("refine_kernel");
   return TAC_OK;
+}
+
+// A candidate to each wave where the documents are short, by the index's mean,
+// and the candidates many: a block of its own for every document of a few
+// tokens costs more than its work.  Call times in us (a block | a wave a
+// candidate; 20,000 candidates, m16, 8 | 32 query tokens): documents of 1 token
+// at dim 64 119 | 43, 153 | 63, at dim 128 256 | 46, 336 | 73; of 1-20 tokens
+// 142 | 70, 198 | 121 and 295 | 93, 384 | 168.  The lines: at 1,000 candidates
+// the block is ahead unless documents have about one token (dim 384, 32 query
+// tokens, 600 candidates: 64 | 34), at 2,000 the wave is until a document has
+// some 2,048 floats (1,536 past five tokens) or 16 tokens (dim 384 at 4.5 tokens
+// and 4,000 candidates 326 | 164, dim 768 at 4.5 tokens 125 | 143, dim 256 at 7.5
+// 83 | 91, dim 32 at 20 40 | 52).
+bool refine_by_wave(const tac_doc_index &ix, uint32_t n_cand) {
+  if (std::max(ix.dim, ix.m) > kRefineWaveFloats) return false;
+  const double mean = ix.n_docs ? (double)ix.n_tokens / (double)ix.n_docs : 0.0;
+  return (n_cand > 512 && mean <= 2.0) ||
+         (n_cand > 1024 && mean < 16.0 && mean * ix.dim <= (mean <= 5.0 ? 2048.0 : 1536.0));
 }
 
 int refine_core(DeviceState &ds, hipStream_t s, const tac_doc_index &ix, const float *d_table,
@@ -2613,9 +2621,28 @@ int refine_core(DeviceState &ds, hipStream_t s, const tac_doc_index &ix, const f
                     (uintptr_t)d_q % 16 == 0;
   // Two tokens a lane when a wave covers at most two (n_q > 16), else one.
   const bool two = fast && n_q > 16;
-  auto *launch = two ? refine_launch<2, true> : fast ? refine_launch<1, true>
-                                                     : refine_launch<1, false>;
-  st = launch(r, d_q, n_q, d_table, d_ids, n_cand, d_scores, first_bad, any_bad, s);
+  const bool by_wave = refine_by_wave(ix, n_cand);
+  // Blocks: up to 512 candidates, or rows past 64 floats: 8 waves and tiles of
+  // 128 tokens, so that a document is one or two steps long; more candidates
+  // fill the chip by themselves and take 4 waves and tiles of 64, whose LDS
+  // lets 5 blocks share a CU.  Call times in us (8 waves x 128 | 4 x 64; 32
+  // query tokens, m16, documents of 1-100 tokens): dim 64 at 250 candidates
+  // 36.2 | 42.7, 500 39.0 | 44.6, 1,000 53.6 | 48.9, 4,000 130 | 106; dim 128
+  // at 1,000 67.9 | 78.3, 4,000 169 | 207.
+  const bool wide = n_cand <= 512 || ix.dim > 64;
+  const uint32_t waves = by_wave ? 4 : wide ? 8 : 4;
+  const uint32_t tile = by_wave ? refine_tile(ix.dim, ix.m, kRefineWaveFloats, 8)
+                                : refine_tile(ix.dim, ix.m, kRefineTileFloats, wide ? 128 : 64);
+  const uint32_t ld = refine_stride(ix.dim, fast);
+  const uint32_t lds = (refine_query_floats(n_q, ld) +
+                        (by_wave ? waves * refine_team_floats(ld, 1, ix.m, tile)
+                                 : refine_team_floats(ld, waves, ix.m, tile))) *
+                       (uint32_t)sizeof(float);
+  auto *launch = two ? (by_wave ? refine_launch<2, true, true> : refine_launch<2, true, false>)
+                 : fast ? (by_wave ? refine_launch<1, true, true> : refine_launch<1, true, false>)
+                        : (by_wave ? refine_launch<1, false, true> : refine_launch<1, false, false>);
+  st = launch(r, d_q, n_q, d_table, d_ids, n_cand, waves, tile, lds, d_scores, first_bad, any_bad,
+              s);
   if (st) return st;
   if (profile) HIP_TRY(hipEventRecord(eb, s));
   HIP_TRY(hipStreamSynchronize(s));

@@ -13,9 +13,15 @@ pytestmark = pytest.mark.gpu
 LENS = [0, 1, 2, 31, 32, 33, 63, 64, 65, 127, 128, 129, 200, 0, 5]
 
 
-def _index(dim, m, ksub, n_q, seed=0):
+# means of 1.2, 1.8 and 9.5 tokens: a wave a candidate past 512 or 1,024
+SHORT = [1, 0, 1, 2, 1, 1, 2, 1, 1, 2]
+SHORTER = [1, 2, 2, 2, 2, 2, 2, 1, 2, 2]
+MIXED = [0, 1, 7, 8, 9, 15, 16, 17, 3, 2, 5, 4, 40, 6]
+
+
+def _index(dim, m, ksub, n_q, seed=0, lens=LENS):
     rng = np.random.default_rng(seed + dim + m + n_q)
-    off = np.concatenate([[0], np.cumsum(LENS)]).astype(np.uint64)
+    off = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint64)
     n = int(off[-1])
     cents = rng.standard_normal((40, dim)).astype(np.float32)
     assign = rng.integers(0, 40, n).astype(np.uint32)
@@ -49,6 +55,50 @@ def test_refine_tile_edges(gpu, dim, m, ksub, n_q, n_cand):
     cand[:ix.n_docs] = np.arange(ix.n_docs)
     got = retrieval.refine(ix, table, q, n_q, cand)
     assert np.array_equal(got.view(np.uint32), want[cand].view(np.uint32))
+
+
+@pytest.mark.parametrize("lens", [SHORT, SHORTER, MIXED])
+@pytest.mark.parametrize("dim,m,ksub,n_q", [
+    (64, 16, 256, 32), (64, 32, 256, 8), (64, 16, 1024, 65), (128, 16, 256, 33), (128, 20, 200, 1),
+    (63, 21, 256, 9), (96, 12, 256, 40), (48, 3, 3, 64), (200, 25, 256, 3), (768, 96, 256, 4),
+    (1536, 16, 256, 2), (1537, 1, 256, 2), (2, 1600, 2, 2)])
+@pytest.mark.parametrize("n_cand", [512, 513, 1025, 70_001])
+def test_refine_short_documents(gpu, lens, dim, m, ksub, n_q, n_cand):
+    """A wave a candidate (four a block, 65,536 of the grid's at once), around
+    the rules that choose it."""
+    ix, table, q = _index(dim, m, ksub, n_q, lens=lens)
+    want = _want(ix, table, q, n_q)
+    cand = np.random.default_rng(2).integers(0, ix.n_docs, n_cand).astype(np.uint32)
+    got = retrieval.refine(ix, table, q, n_q, cand)
+    assert np.array_equal(got.view(np.uint32), want[cand].view(np.uint32))
+
+
+@pytest.mark.parametrize("dim", [64, 96])
+@pytest.mark.parametrize("where", ["code", "id", "count", "doc"])
+def test_refine_short_documents_corrupt(gpu, dim, where):
+    """The first failing candidate of many is reported, whichever wave meets it;
+    a clean call works afterwards."""
+    m, ksub, n_q, n_cand = 16, 200, 20, 3000
+    ix, table, q = _index(dim, m, ksub, n_q, seed=5, lens=MIXED)
+    bad, d = ix.doc_payload.copy(), 7  # 17 tokens
+    lo = int(ix.doc_index[d])
+    if where == "code":
+        bad[lo + 4 + 4 * 17 + 17 * m - 1] = 250
+    elif where == "id":
+        bad[lo + 4 + 4 * 16] = 40
+    elif where == "count":
+        bad[lo] = 16
+    ixb = retrieval.DocIndex(dim, m, ksub, ix.centroids, ix.doc_index, bad, ix.doc_token_offsets,
+                             ix.residual_norms)
+    cand = np.full(n_cand, 3, np.uint32)
+    cand[[1234, 2900, 2999]] = ix.n_docs if where == "doc" else d
+    kind = errors.DocOutOfRange if where == "doc" else errors.DocLayoutCorrupt
+    with pytest.raises(kind):
+        retrieval.refine(ixb, table, q, n_q, cand)
+    assert lib.tac_gpu_last_error().endswith(b"candidate 1234")
+    cand[:] = np.arange(n_cand) % ix.n_docs
+    got = retrieval.refine(ix, table, q, n_q, cand)
+    assert np.array_equal(got.view(np.uint32), _want(ix, table, q, n_q)[cand].view(np.uint32))
 
 
 @pytest.mark.parametrize("shift", [1, 2, 4])
