@@ -10,6 +10,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "pq_kernels.hpp"
+
 namespace tacgpu {
 
 constexpr int kResBlock = 256;  // threads per residual block
@@ -296,12 +298,13 @@ __device__ __forceinline__ void doc_copy(uint32_t lane, uint64_t lo, uint64_t n_
 }
 
 // Phase 3: adds each scan block's carry-in to the document's offset and writes
-// the layouts, one wave per document or slice (grid-stride).
+// the layouts, one wave per slice or per `group` (at most 64) consecutive
+// documents, whose offsets its lanes load at once (grid-stride).
 __global__ __launch_bounds__(256) void doc_write_kernel(
     const uint64_t* __restrict__ doc_offsets, uint64_t n_docs, const uint32_t* __restrict__ assign,
     const uint8_t* __restrict__ codes, uint32_t m, uint32_t cb,
     const uint64_t* __restrict__ sums, uint64_t* __restrict__ doc_index,
-    uint8_t* __restrict__ payload, const DocState* __restrict__ st,
+    uint8_t* __restrict__ payload, uint32_t group, const DocState* __restrict__ st,
     const DocSlice* __restrict__ slices) {
   const uint32_t lane = threadIdx.x % 64;
   const uint64_t waves = (uint64_t)gridDim.x * (blockDim.x / 64);
@@ -315,12 +318,23 @@ __global__ __launch_bounds__(256) void doc_write_kernel(
     doc_copy(lane, lo, n_d, sl.first, k1,
              payload + sl.at + sums[sl.doc / (kScanBlock * kScanPer)], assign, codes, m, cb);
   }
-  for (uint64_t d = wave; d < n_docs; d += waves) {
-    const uint64_t lo = doc_offsets[d], n_d = doc_offsets[d + 1] - lo;
-    const uint64_t at = doc_index[d] + sums[d / (kScanBlock * kScanPer)];
-    if (lane == 0) doc_index[d] = at;
-    if (go && n_d <= kDocSlice)
-      doc_copy(lane, lo, n_d, 0, n_d, payload + at, assign, codes, m, cb);
+  for (uint64_t base = wave * group; base < n_docs; base += waves * group) {
+    const uint32_t cnt = n_docs - base < group ? (uint32_t)(n_docs - base) : group;
+    const uint64_t d = base + lane;
+    uint64_t lo = 0, n_d = 0, at = 0;
+    if (lane < cnt) {
+      lo = doc_offsets[d];
+      n_d = doc_offsets[d + 1] - lo;
+      at = doc_index[d] + sums[d / (kScanBlock * kScanPer)];
+      doc_index[d] = at;
+    }
+    if (!go) continue;
+    for (uint32_t k = 0; k < cnt; ++k) {
+      const uint64_t n_k = readlane_u64(n_d, k);
+      if (n_k <= kDocSlice)
+        doc_copy(lane, readlane_u64(lo, k), n_k, 0, n_k, payload + readlane_u64(at, k), assign,
+                 codes, m, cb);
+    }
   }
 }
 

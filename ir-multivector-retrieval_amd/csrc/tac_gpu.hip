@@ -2444,6 +2444,18 @@ namespace {
 
 uint64_t align8_host(uint64_t x) { return (x + 7u) & ~(uint64_t)7u; }
 
+// Consecutive documents that a wave of doc_write_kernel takes: one until the
+// waves fill the chip twice, then by their number up to 16, so that one load
+// fetches the offsets of all.  Call times in us, 1 | 2 | 4 | 8 | 16 | 32 to a wave
+// (m16): 1.5M documents of one token 389 | 299 | 242 | 213 | 202 | 199, 143,000
+// of 1-20 62 | 52 | 48 | 48 | 53 | 56, 30,000 of 1-100 37 | 36 | 35 | 42 | 54,
+// 40,000 of 1-300 61 | 62 | 69 | 76.
+uint32_t doc_group(uint64_t n_docs) {
+  uint32_t g = 1;
+  while (g < 16 && n_docs >= 32768ull * g) g <<= 1;
+  return g;
+}
+
 int doc_layouts_core(DeviceState &ds, hipStream_t s, const uint64_t *d_off, uint64_t n_docs,
                      uint64_t n_tokens, const uint32_t *d_assign, const uint8_t *d_codes,
                      uint32_t m, uint32_t cb, uint64_t *d_index, uint8_t *d_payload,
@@ -2474,11 +2486,12 @@ int doc_layouts_core(DeviceState &ds, hipStream_t s, const uint64_t *d_off, uint
                                                            d_index, sums, state, slices);
   doc_sums_scan_kernel<<<1, kScanBlock, 0, s>>>(sums, (uint32_t)nb, d_index, n_docs, payload_len,
                                                 state, ds.host_words);
-  const uint64_t waves_wanted =
-      std::min<uint64_t>(std::max(n_docs, doc_slices_most(n_tokens)), 1ull << 20);
+  const uint32_t group = doc_group(n_docs);
+  const uint64_t waves_wanted = std::min<uint64_t>(
+      std::max((n_docs + group - 1) / group, doc_slices_most(n_tokens)), 1ull << 20);
   const unsigned blocks = (unsigned)((waves_wanted + 3) / 4);
   doc_write_kernel<<<blocks, 256, 0, s>>>(d_off, n_docs, d_assign, d_codes, m, cb, sums, d_index,
-                                          d_payload, state, slices);
+                                          d_payload, group, state, slices);
   LAUNCH_TRY("doc layout kernels");
   HIP_TRY(hipStreamSynchronize(s));
   const uint32_t *host = ds.host_words;

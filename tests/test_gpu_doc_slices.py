@@ -31,6 +31,17 @@ def test_slices_and_scan_blocks(gpu, lens):
     _check(lens, 16, 1, seed=len(lens))
 
 
+@pytest.mark.parametrize("n_docs", [32_767, 32_768, 65_537, 131_073, 262_143, 262_144, 300_007])
+def test_groups_of_documents(gpu, n_docs):
+    """1 to 16 documents a wave (by 32,768, 65,536, 131,072 and 262,144), the
+    last group ragged, with documents around the slices' 512 tokens among them."""
+    rng = np.random.default_rng(n_docs)
+    lens = rng.integers(0, 4, n_docs)
+    lens[rng.integers(0, n_docs, 60)] = rng.integers(500, 1030, 60)
+    lens[[0, 15, 16, -2, -1]] = [512, 513, 600, 513, 512]
+    _check(lens, 5, 1, seed=n_docs)
+
+
 def test_layout_errors_leave_the_state_clean(gpu):
     """A short payload and unsound offsets with long documents, then a good call."""
     n = 3000
