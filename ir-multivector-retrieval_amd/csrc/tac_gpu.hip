@@ -608,10 +608,28 @@ inline uint32_t list_split(uint32_t K) {
 // vectors a thread | this kernel: m32 dsub 2 K256 at 1 row 33 | 9, 1,000
 // 44 | 11, 16,000 60 | 32; m16 dsub 4 K1024 at 180 rows 120 | 13, 16,000
 // 210 | 76), and to 8,192 at 5-8, where the matrix-core screen takes over
-// (m16 dsub 8 K256 at 180 rows 30 | 12, 1,000 48 | 12, 8,000 67 | 26).
+// (m16 dsub 8 K256 at 180 rows 30 | 12, 1,000 48 | 12, 8,000 67 | 26).  Many
+// subspaces fill the chip by themselves, and the pruned searches are then ahead
+// at fewer rows, the sooner the longer a scan is: from encode_small_cells
+// row-subspaces (K256: dsub 1 m192 at 16,000 rows 178 | 123; dsub 2 m128 at
+// 12,000 98 | 96, m192 at 16,000 130 | 153, with K1024 627 | 496; dsub 3 m96 at
+// 12,000 94 | 86, m128 at 12,000 96 | 109; dsub 4 m64 at 16,000 96 | 88, m128 at
+// 8,000 84 | 86, at 12,000 109 | 120; at 8,192 rows dsub 8 m64 93 | 81, m96 87 |
+// 112, with K64 m192 72 | 71, with K1024 m96 487 | 417, m128 529 | 548, dsub 6
+// m96 286 | 318).
 constexpr uint64_t kEncodeSmallRows = 16384, kEncodeSmallRowsWide = 8192;
-inline bool encode_is_small(uint64_t n, uint32_t D) {
-  return D <= 4 ? n < kEncodeSmallRows : n <= kEncodeSmallRowsWide;
+inline uint64_t encode_small_cells(uint32_t K, uint32_t D) {
+  switch (D) {
+    case 1: return 3u << 20;
+    case 2: return K <= 256 ? 7u << 18 : 3u << 20;
+    case 3: return 5u << 18;
+    case 4: return 1u << 20;
+    default: return K <= 64 ? 3u << 19 : K <= 256 ? 1u << 19 : 3u << 18;
+  }
+}
+inline bool encode_is_small(uint64_t n, uint32_t M, uint32_t K, uint32_t D) {
+  return (D <= 4 ? n < kEncodeSmallRows : n <= kEncodeSmallRowsWide) &&
+         n * M <= encode_small_cells(K, D);
 }
 // Its lanes per vector: 16 while the rows are few for the length of a scan
 // (16 | 4 lanes: m16 dsub 4 K256 at 180 rows 9.9 | 11.5 us, 4,000 15.1 |
@@ -991,7 +1009,7 @@ struct Launch {
   template <typename CodeT>
   static int encode(const float *x, const float *cb, CodeT *codes, uint64_t n, uint32_t dim,
                     uint32_t M, uint32_t K, unsigned long long *rescans, hipStream_t s) {
-    if (encode_is_small(n, D))
+    if (encode_is_small(n, M, K, D))
       return encode_wide_lanes(n, M, K, D)
                  ? encode_small<16, CodeT>(x, cb, codes, n, dim, M, K, s)
                  : encode_small<4, CodeT>(x, cb, codes, n, dim, M, K, s);
@@ -1706,7 +1724,7 @@ int encode_core(DeviceState &ds, hipStream_t s, const float *d_x, uint64_t n, ui
                                              n, dim, M, K, L, rescans, s));
     }
   } else if (D >= 5 && D <= 8 && screen_wanted(K) && n <= 0xFFFFFFFFull &&
-             !encode_is_small(n, D)) {
+             !encode_is_small(n, M, K, D)) {
     if ((st = ensure(ds, ds.cand_defer, (size_t)2 * M * n * sizeof(uint32_t))) ||
         (st = ensure(ds, ds.cand_count, (size_t)M * sizeof(uint32_t))))
       return st;
@@ -2120,7 +2138,7 @@ int tac_pq_encode_device_noalloc(const float *d_residuals, uint64_t n, uint32_t 
   // Sub-dimensions 5-8 with ksub <= 256: the matrix-core screen, its
   // deferred list (one word per row and subspace) and count in the scratch,
   // in batches of whole sort tiles that fit.
-  if (D >= 5 && D <= 8 && screen_wanted(ksub) && !encode_is_small(n, D)) {
+  if (D >= 5 && D <= 8 && screen_wanted(ksub) && !encode_is_small(n, m, ksub, D)) {
     uint32_t *dcount = reinterpret_cast<uint32_t *>(take((size_t)m * sizeof(uint32_t)));
     const size_t left = off < kNoAllocScratchBytes ? kNoAllocScratchBytes - off : 0;
     uint64_t sb = left / (sizeof(uint32_t) * (size_t)m) / kSortTile * kSortTile;

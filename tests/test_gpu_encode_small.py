@@ -33,6 +33,28 @@ def test_rows_and_lane_widths(gpu, dsub, m, ksub, n):
     assert np.array_equal(_encode(x, cb, m, ksub), want)
 
 
+@pytest.mark.parametrize("dsub,m,ksub,n,small", [
+    (1, 256, 64, 12_288, True), (1, 256, 64, 12_289, False), (2, 192, 64, 9557, True),
+    (2, 192, 64, 9558, False), (3, 81, 1024, 16_181, True), (3, 81, 1024, 16_182, False),
+    (4, 128, 256, 8192, True), (4, 128, 256, 8193, False), (8, 96, 256, 5461, True),
+    (8, 96, 256, 5462, False), (5, 193, 64, 8149, True), (5, 193, 64, 8150, False),
+    (6, 129, 300, 6096, True), (6, 129, 300, 6097, False), (2, 193, 300, 16_299, True),
+    (2, 193, 300, 16_300, False)])
+def test_many_subspaces(gpu, dsub, m, ksub, n, small):
+    """Around the row-subspaces past which the pruned searches take over (by
+    sub-dimension and codewords)."""
+    rng = np.random.default_rng(m + n)
+    x = (rng.standard_normal((n, m * dsub)) * 0.2).astype(np.float32)
+    cb = (rng.standard_normal((m, ksub, dsub)) * 0.2).astype(np.float32)
+    device.profile_enable(True)
+    device.profile_kernels(reset=True)
+    got = _encode(x, cb, m, ksub)
+    names = " ".join(device.profile_kernels(reset=True))
+    device.profile_enable(False)
+    assert ("encode_small_kernel" in names) == small
+    assert np.array_equal(got, orc.pq_encode(x, m * dsub, m, ksub, cb, n_threads=8))
+
+
 @pytest.mark.parametrize("dsub", [2, 4, 8])
 @pytest.mark.parametrize("lanes", [4, 16])
 def test_special_values_and_lane_count(gpu, dsub, lanes):
