@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 from oracle import binding as orc
-from tac_gpu import device, errors, kmeans, pq, synth
+from tac_gpu import device, errors, kmeans, lib, pq, synth
 
 NEVER = float("-inf")
 pytestmark = pytest.mark.gpu
@@ -300,7 +300,38 @@ def _encode_both(x, cb, m, ksub):
     return got, orc.pq_encode(x, dim, m, ksub, cb)
 
 
-def test_pruned_search_near_ties_across_blocks(gpu):
+def _check_pruned(x, cb, m, ksub, monkeypatch):
+    """The same rows, repeated to 16,500, through encode_kernel: the full search
+    that the environment asks for, and past 256 codewords (the book repeated)
+    the entry that allocates nothing.  The kernel that ran is checked by name."""
+    dim = x.shape[1]
+    n = 16_500
+    x = np.ascontiguousarray(x[np.arange(n) % x.shape[0]])
+    cb = np.ascontiguousarray(cb, np.float32)
+
+    def ran(call):
+        device.profile_enable(True)
+        device.profile_kernels(reset=True)
+        codes = call()
+        names = set(device.profile_kernels(reset=True))
+        device.profile_enable(False)
+        assert any(k.startswith("encode_kernel<") for k in names), names
+        assert not any("small" in k or "cand" in k or "cell" in k for k in names), names
+        return codes
+
+    monkeypatch.setenv("TAC_GPU_FULL_SEARCH", "1")
+    got = ran(lambda: pq.PQ(dim, dim // m, cb.reshape(-1), m, ksub).encode_many(x))
+    assert np.array_equal(got, orc.pq_encode(x, dim, m, ksub, cb, n_threads=16))
+    monkeypatch.delenv("TAC_GPU_FULL_SEARCH")
+    wide = np.ascontiguousarray(cb[:, np.arange(520) % ksub])
+    dx, dcb = device.DeviceArray.from_host(x), device.DeviceArray.from_host(wide)
+    dc = device.DeviceArray((n, m), np.uint16)
+    errors.check(lib.tac_pq_encode_device_noalloc(dx.ptr, n, dim, m, 520, dcb.ptr, dc.ptr, None))
+    device.synchronize()
+    assert np.array_equal(dc.to_host(), orc.pq_encode(x, dim, m, 520, wide, n_threads=16))
+
+
+def test_pruned_search_near_ties_across_blocks(gpu, monkeypatch):
     # Codewords 3 and 200 (different blocks of 8) sit symmetrically around
     # every vector's sub-vector, so their distances tie in exact arithmetic
     # and differ by at most rounding; codeword 77 is a few ulps farther.
@@ -318,18 +349,20 @@ def test_pruned_search_near_ties_across_blocks(gpu):
     x += (rng.integers(-2, 3, x.shape) * np.float32(1e-9)).astype(np.float32)
     got, ref = _encode_both(x, cb, m, ksub)
     assert np.array_equal(got, ref)
+    _check_pruned(x, cb, m, ksub, monkeypatch)
 
 
-def test_pruned_search_duplicate_codewords_across_blocks(gpu):
+def test_pruned_search_duplicate_codewords_across_blocks(gpu, monkeypatch):
     rng = np.random.default_rng(32)
     x = (rng.standard_normal((3000, 64)) * 0.2).astype(np.float32)
     cb = (rng.standard_normal((16, 256, 4)) * 0.2).astype(np.float32)
     cb[:, 8 * np.arange(32) + 5] = cb[:, 5:6]  # one codeword repeated in every block
     got, ref = _encode_both(x, cb, 16, 256)
     assert np.array_equal(got, ref)
+    _check_pruned(x, cb, 16, 256, monkeypatch)
 
 
-def test_pruned_search_wide_bounds(gpu):
+def test_pruned_search_wide_bounds(gpu, monkeypatch):
     # A few far-away codewords make cmax large, so the gap test is loose and
     # many searches fall back to the full scan; results must not change.
     rng = np.random.default_rng(33)
@@ -338,9 +371,10 @@ def test_pruned_search_wide_bounds(gpu):
     cb[:, 255] = 1e6
     got, ref = _encode_both(x, cb, 16, 256)
     assert np.array_equal(got, ref)
+    _check_pruned(x, cb, 16, 256, monkeypatch)
 
 
-def test_pruned_search_non_finite_values(gpu):
+def test_pruned_search_non_finite_values(gpu, monkeypatch):
     rng = np.random.default_rng(34)
     x = (rng.standard_normal((700, 64)) * 0.2).astype(np.float32)
     cb = (rng.standard_normal((16, 64, 4)) * 0.2).astype(np.float32)
@@ -352,14 +386,16 @@ def test_pruned_search_non_finite_values(gpu):
     x[7, :] = np.float32(2e38)
     got, ref = _encode_both(x, cb, 16, 64)
     assert np.array_equal(got, ref)
+    _check_pruned(x, cb, 16, 64, monkeypatch)
 
 
 @pytest.mark.parametrize("ksub", [1, 2, 7, 8, 9, 100])
-def test_pruned_search_small_and_ragged_ksub(gpu, ksub):
+def test_pruned_search_small_and_ragged_ksub(gpu, monkeypatch, ksub):
     x = _workload_rows(3001, seed=ksub)
     cb = synth.gauss_codebooks(ksub, 16, ksub, 4, 0.1)
     got, ref = _encode_both(x, cb, 16, ksub)
     assert np.array_equal(got, ref)
+    _check_pruned(x, cb, 16, ksub, monkeypatch)
 
 
 def test_train_with_duplicate_init_codewords_across_blocks(gpu):

@@ -158,8 +158,9 @@ def test_encode_ties_and_non_finite(gpu, monkeypatch):
 @pytest.mark.parametrize("scale", [1e-25, 1e15, 1e20])
 def test_encode_magnitudes(gpu, monkeypatch, scale):
     rng = np.random.default_rng(29)
-    x = (rng.standard_normal((6000, 64)) * scale).astype(np.float32)
+    x = (rng.standard_normal((12_345, 64)) * scale).astype(np.float32)
     cb = synth.shuffle_init(x, 8, 256, 6).reshape(-1)
     prof = _check_encode(x, 64, 8, 256, cb, monkeypatch)
+    assert prof.screen_vectors == 8 * x.shape[0]
     if scale < 1e-18 or scale > 1e18:
         assert prof.screen_deferred == prof.screen_vectors
