@@ -4,7 +4,6 @@ import ctypes
 
 import numpy as np
 import pytest
-import torch
 
 from tac_gpu import errors, lib, pq
 
@@ -40,20 +39,26 @@ def test_bad_code_leaves_the_output(gpu, n):
 
 @pytest.mark.parametrize("floats", [524_287, 1_310_721, 4_194_305, 9_000_001])
 def test_pinned_output(gpu, floats):
+    """Outputs inside a pinned allocation, from the runtime the library uses."""
     rng = np.random.default_rng(floats)
     cb = rng.standard_normal(256).astype(np.float32)
     codes = rng.integers(0, 256, (floats, 1)).astype(np.uint8)
-    out = torch.full((floats + 64,), 7.0, pin_memory=True)
+    mem = ctypes.c_void_p()
+    assert lib.hipHostMalloc(ctypes.byref(mem), ctypes.c_size_t(4 * (floats + 64)), 0) == 0
+    try:
+        out = np.ctypeslib.as_array(ctypes.cast(mem, ctypes.POINTER(ctypes.c_float)), (floats + 64,))
 
-    def call():
-        p = [ctypes.c_void_p(a.ctypes.data) for a in (codes, cb)]
-        return lib.tac_pq_decode(p[0], floats, 1, 1, 256, p[1], ctypes.c_void_p(out.data_ptr() + 128))
+        def call(ksub):
+            p = [ctypes.c_void_p(a.ctypes.data) for a in (codes, cb, out[32:])]
+            return lib.tac_pq_decode(p[0], floats, 1, 1, ksub, p[1], p[2])
 
-    for _ in range(2):
-        assert call() == 0
-        assert np.array_equal(out[32:32 + floats].numpy(), cb[codes[:, 0]])
-        assert (out[:32] == 7.0).all() and (out[32 + floats:] == 7.0).all()
-    out[:] = 7.0
-    p = [ctypes.c_void_p(a.ctypes.data) for a in (codes, cb)]
-    status = lib.tac_pq_decode(p[0], floats, 1, 1, 100, p[1], ctypes.c_void_p(out.data_ptr()))
-    assert status == errors.InvalidArgument.status and (out == 7.0).all()
+        for _ in range(2):
+            out[:] = 7.0
+            assert call(256) == 0
+            assert np.array_equal(out[32:32 + floats], cb[codes[:, 0]])
+            assert (out[:32] == 7.0).all() and (out[32 + floats:] == 7.0).all()
+        out[:] = 7.0
+        assert call(100) == errors.InvalidArgument.status and (out == 7.0).all()
+    finally:
+        del out
+        lib.hipHostFree(mem)
