@@ -174,6 +174,18 @@ int ensure(DeviceState &ds, Buffer &b, size_t bytes) {
   return TAC_OK;
 }
 
+// A buffer whose contents last from call to call: allocated and filled once.  A
+// failed fill leaves no buffer, so that the next call fills it.
+int ensure_filled(DeviceState &ds, Buffer &b, size_t bytes, int value, hipStream_t s) {
+  if (b.ptr) return TAC_OK;
+  if (int st = ensure(ds, b, bytes)) return st;
+  const hipError_t e = hipMemsetAsync(b.ptr, value, bytes, s);
+  if (e == hipSuccess) return TAC_OK;
+  (void)hipFree(b.ptr);
+  b = Buffer{};
+  return hip_status("hipMemsetAsync(workspace)", e);
+}
+
 constexpr size_t kStageChunk = 8u << 20;  // bytes per staged copy
 constexpr size_t kStageMin = 32u << 20;   // smaller uploads copy from pageable memory directly
 
@@ -2489,12 +2501,9 @@ int doc_layouts_core(DeviceState &ds, hipStream_t s, const uint64_t *d_off, uint
   if (nb > 0x7FFFFFFFull) return TAC_ERR_UNSUPPORTED;
   int st;
   if ((st = host_words(ds)) || (st = ensure(ds, ds.scan_sums, (size_t)nb * sizeof(uint64_t))) ||
-      (st = ensure(ds, ds.doc_slices, (size_t)doc_slices_most(n_tokens) * sizeof(DocSlice))))
+      (st = ensure(ds, ds.doc_slices, (size_t)doc_slices_most(n_tokens) * sizeof(DocSlice))) ||
+      (st = ensure_filled(ds, ds.doc_state, sizeof(DocState), 0, s)))
     return st;
-  if (!ds.doc_state.ptr) {
-    if ((st = ensure(ds, ds.doc_state, sizeof(DocState)))) return st;
-    HIP_TRY(hipMemsetAsync(ds.doc_state.ptr, 0, sizeof(DocState), s));
-  }
   uint64_t *sums = as<uint64_t>(ds.scan_sums);
   DocState *state = as<DocState>(ds.doc_state);
   DocSlice *slices = as<DocSlice>(ds.doc_slices);
@@ -2631,11 +2640,9 @@ int refine_core(DeviceState &ds, hipStream_t s, const tac_doc_index &ix, const f
   // The failing candidate's word stays all ones between calls: only a call
   // that raised the host flag has to read it back and restore it.
   int st;
-  if ((st = host_words(ds))) return st;
-  if (!ds.io_x3.ptr) {
-    if ((st = ensure(ds, ds.io_x3, sizeof(unsigned long long)))) return st;
-    HIP_TRY(hipMemsetAsync(ds.io_x3.ptr, 0xFF, sizeof(unsigned long long), s));
-  }
+  if ((st = host_words(ds)) ||
+      (st = ensure_filled(ds, ds.io_x3, sizeof(unsigned long long), 0xFF, s)))
+    return st;
   unsigned long long *first_bad = as<unsigned long long>(ds.io_x3);
   uint32_t *any_bad = ds.host_words;
   *any_bad = 0;
