@@ -154,7 +154,7 @@ TAC_HD inline uint64_t fold_chunk_q(Acc s, const FoldChunk& ch) {
 // (alone past the binade) makes its candidate unusable, so the others fit.
 struct FoldSlim {
   uint32_t q[kFoldCands];
-  uint32_t tag;  // exponent bits of candidate 0; from bit 8 the usable candidates
+  uint32_t tag;  // exponent bits of candidate 0; from bit 8 the usable candidates; from 16 free
 };
 constexpr uint32_t kFoldSlimBad = ~0u;
 

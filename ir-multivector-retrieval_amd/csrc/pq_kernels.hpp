@@ -1271,8 +1271,8 @@ constexpr uint32_t kFoldStaged = 32;  // chunks whose terms are staged
 
 struct FoldStage {
   __attribute__((aligned(16))) float terms[kFoldStaged + 1][kFoldChunk];  // the last: unstaged
+  // tag from bit 16: the chunk's row of `terms`, or kFoldStaged
   __attribute__((aligned(16))) FoldSlim chunk[kFoldWindow];
-  uint8_t slot[kFoldWindow];  // row of `terms`, or kFoldStaged
   uint16_t chunk_of[kFoldStaged];
   uint32_t n_slots;
 };
@@ -1319,8 +1319,7 @@ __device__ inline float fold_apply_block(const float* __restrict__ em, uint64_t 
       const uint32_t j = w0 + i;
       const float a = (float)pre[j];
       const float b = j + 1 < nc ? (float)pre[j + 1] : a;
-      const FoldSlim ch = fold_slim(cm[j]);
-      st.chunk[i] = ch;
+      FoldSlim ch = fold_slim(cm[j]);
       const bool clean = fold_is_normal_positive(a) && fold_slim_q(a, ch) != kFoldSlimBad;
       uint32_t slot = kFoldStaged;
       if (!clean || fold_exponent(a) != fold_exponent(b)) {
@@ -1330,7 +1329,8 @@ __device__ inline float fold_apply_block(const float* __restrict__ em, uint64_t 
           st.chunk_of[at] = (uint16_t)i;
         }
       }
-      st.slot[i] = (uint8_t)slot;
+      ch.tag |= slot << 16;
+      st.chunk[i] = ch;
     }
     __syncthreads();
     const uint32_t ns = st.n_slots < kFoldStaged ? st.n_slots : kFoldStaged;
@@ -1355,36 +1355,44 @@ __device__ inline float fold_apply_block(const float* __restrict__ em, uint64_t 
     }
     __syncthreads();
     if (w == 0) {
-      for (uint32_t i = 0; i < wn;) {
-        const uint32_t cnt = wn - i < kWave ? wn - i : kWave;
-        uint32_t b = 0;  // chunks applied through the prefix sum
-        if (fold_is_normal_positive(s)) {
-          const uint32_t m = (uint32_t)fold_units(s);
-          const FoldSlim ch = st.chunk[i + (lane < cnt ? lane : 0)];
-          const uint32_t Q = fold_slim_q(s, ch);
-          const bool ok = Q != kFoldSlimBad;  // then at most 2^24: 64 of them fit 32 bits
-          const uint32_t P = wave_inclusive_sum_u32(ok ? Q : 0u);
-          const uint64_t bad = __ballot(lane < cnt && !(ok && fold_run_fits<float>(m, P)));
-          b = bad ? (uint32_t)__builtin_ctzll(bad) : cnt;
-          if (b > 0)
-            s = fold_with_units(s, m + (uint32_t)__builtin_amdgcn_readlane((int)P, (int)b - 1));
-        }
-        i += b;
-        if (b < cnt) {
-          const uint32_t j = w0 + i, slot = st.slot[i];
-          if (slot == kFoldStaged) {
-            // Unexpected chunks come in runs (a long stretch of ties): the
-            // next one's terms are loaded while this one's are added.
-            if (next != j) fetch(j);
-            wave_lds_sync();
-#pragma unroll
-            for (uint32_t t = 0; t < kPer; ++t) st.terms[slot][t * kWave + lane] = ahead[t];
-            wave_lds_sync();
-            if (j + 1 < nc) fetch(j + 1);
+      FoldSlim ch = st.chunk[lane];
+      for (uint32_t g = 0; g < wn; g += kWave) {  // a chunk a lane
+        const uint32_t cnt = wn - g < kWave ? wn - g : kWave;
+        const uint32_t ahead_at = g + kWave + lane;
+        const FoldSlim later = st.chunk[ahead_at < kFoldWindow ? ahead_at : lane];
+        for (uint32_t at = 0; at < cnt;) {  // chunks below g + at are applied
+          uint32_t b = at;
+          if (fold_is_normal_positive(s)) {
+            const uint32_t m = (uint32_t)fold_units(s);
+            const bool in = lane >= at && lane < cnt;
+            const uint32_t Q = fold_slim_q(s, ch);
+            const bool ok = Q != kFoldSlimBad;  // then at most 2^24: 64 of them fit 32 bits
+            const uint32_t P = wave_inclusive_sum_u32(in && ok ? Q : 0u);
+            const uint64_t bad = __ballot(in && !(ok && fold_run_fits<float>(m, P)));
+            b = bad ? (uint32_t)__builtin_ctzll(bad) : cnt;
+            if (b > at)
+              s = fold_with_units(s, m + (uint32_t)__builtin_amdgcn_readlane((int)P, (int)b - 1));
           }
-          s = fold_chunk_terms(s, st.terms[slot]);
-          ++i;
+          at = b;
+          if (b < cnt) {
+            const uint32_t j = w0 + g + b;
+            const uint32_t slot =
+                (uint32_t)__builtin_amdgcn_readlane((int)ch.tag, (int)b) >> 16;
+            if (slot == kFoldStaged) {
+              // Unexpected chunks come in runs (a long stretch of ties): the
+              // next one's terms are loaded while this one's are added.
+              if (next != j) fetch(j);
+              wave_lds_sync();
+#pragma unroll
+              for (uint32_t t = 0; t < kPer; ++t) st.terms[slot][t * kWave + lane] = ahead[t];
+              wave_lds_sync();
+              if (j + 1 < nc) fetch(j + 1);
+            }
+            s = fold_chunk_terms(s, st.terms[slot]);
+            ++at;
+          }
         }
+        ch = later;
       }
     }
     __syncthreads();
