@@ -257,14 +257,6 @@ __global__ __launch_bounds__(512, 4) void refine_kernel(
   const uint32_t teams = WAVES ? blockDim.x / 64 : 1, team = WAVES ? threadIdx.x / 64 : 0;
   const uint32_t W = WAVES ? 1 : blockDim.x / 64, w = WAVES ? 0 : threadIdx.x / 64;
   const uint32_t tid = WAVES ? lane : threadIdx.x, nt = WAVES ? 64 : blockDim.x;
-  auto team_any = [](bool v) -> bool {  // and the team's LDS accesses ordered
-    if constexpr (WAVES) {
-      wave_lds_sync();
-      return __any(v);
-    } else {
-      return __syncthreads_or(v);
-    }
-  };
   const uint32_t ld = refine_stride(ix.dim, FAST);
   const uint32_t QP = refine_qp(n_q), S = 64 / QP;
   const uint32_t slot = lane / QP, qi = lane % QP;
@@ -368,7 +360,9 @@ __global__ __launch_bounds__(512, 4) void refine_kernel(
             rows[s * ld + d] = ix.centroids[(uint64_t)cid * ix.dim + d];
           }
         }
-        if (team_any(bad)) {  // also: the rows (and the queries) are staged
+        if constexpr (WAVES) wave_lds_sync();
+        // also: the rows (and the queries) are staged
+        if (WAVES ? __any(bad) : __syncthreads_or(bad)) {
           st = kRefineLayoutCorrupt;
           break;
         }
@@ -402,7 +396,9 @@ __global__ __launch_bounds__(512, 4) void refine_kernel(
               bk = k0 + t[r];
             }
         }
-        if (team_any(bad)) {  // also: the rows may be overwritten
+        if constexpr (WAVES) wave_lds_sync();
+        // also: the rows may be overwritten
+        if (WAVES ? __any(bad) : __syncthreads_or(bad)) {
           st = kRefineLayoutCorrupt;
           break;
         }
