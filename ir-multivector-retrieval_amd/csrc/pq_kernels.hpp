@@ -578,22 +578,28 @@ __global__ __launch_bounds__(kBlock) void scan_apply_kernel(
   const uint32_t c0 = threadIdx.x * per_c;
   const uint32_t nq = c0 < K ? (K - c0 < per_c ? K - c0 : per_c) : 0u;
   uint32_t tot[4] = {0, 0, 0, 0}, before[PER] = {};
-  // All ranges' sums are loaded before the first is added: one after another,
+  // The ranges' sums are loaded before the first is added: one after another,
   // the ranges were up to 32 round trips (10.8 us at 58 tiles of 8 subspaces,
-  // 4.9 now).
-  uint32_t sum[kScanRanges][PER];
+  // 4.9 now).  With four codes a lane they would fill 128 registers; the kernel
+  // is then no shorter, and its blocks take the place of the other training
+  // stream's (K1024, m32 dsub 2: 8 iterations of 500,000 rows 4,820 us with all
+  // loaded at once, 4,490 one by one, of 400,000 4,130 and 3,940).
+  constexpr uint32_t kBatch = PER >= 4 ? 1 : kScanRanges;
+  for (uint32_t g0 = 0; g0 < G; g0 += kBatch) {
+    uint32_t sum[kBatch][PER];
 #pragma unroll
-  for (uint32_t gg = 0; gg < kScanRanges; ++gg)
+    for (uint32_t u = 0; u < kBatch; ++u)
 #pragma unroll
-    for (uint32_t q = 0; q < PER; ++q)
-      sum[gg][q] = gg < G && q < nq ? pm[(uint64_t)gg * K + c0 + q] : 0u;
+      for (uint32_t q = 0; q < PER; ++q)
+        sum[u][q] = g0 + u < G && q < nq ? pm[(uint64_t)(g0 + u) * K + c0 + q] : 0u;
 #pragma unroll
-  for (uint32_t gg = 0; gg < kScanRanges; ++gg)
+    for (uint32_t u = 0; u < kBatch; ++u)
 #pragma unroll
-    for (uint32_t q = 0; q < PER; ++q) {
-      before[q] += gg < g ? sum[gg][q] : 0u;
-      tot[q] += sum[gg][q];
-    }
+      for (uint32_t q = 0; q < PER; ++q) {
+        before[q] += g0 + u < g ? sum[u][q] : 0u;
+        tot[q] += sum[u][q];
+      }
+  }
   uint32_t local = 0;
 #pragma unroll
   for (uint32_t q = 0; q < PER; ++q) local += tot[q];
