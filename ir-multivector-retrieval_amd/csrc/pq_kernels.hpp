@@ -582,22 +582,29 @@ __global__ __launch_bounds__(kBlock) void scan_apply_kernel(
   // the ranges were up to 32 round trips (10.8 us at 58 tiles of 8 subspaces,
   // 4.9 now).  With four codes a lane they would fill 128 registers; the kernel
   // is then no shorter, and its blocks take the place of the other training
-  // stream's (K1024, m32 dsub 2: 8 iterations of 500,000 rows 4,820 us with all
-  // loaded at once, 4,490 one by one, of 400,000 4,130 and 3,940).
-  constexpr uint32_t kBatch = PER >= 4 ? 1 : kScanRanges;
-  for (uint32_t g0 = 0; g0 < G; g0 += kBatch) {
-    uint32_t sum[kBatch][PER];
-#pragma unroll
-    for (uint32_t u = 0; u < kBatch; ++u)
-#pragma unroll
-      for (uint32_t q = 0; q < PER; ++q)
-        sum[u][q] = g0 + u < G && q < nq ? pm[(uint64_t)(g0 + u) * K + c0 + q] : 0u;
-#pragma unroll
-    for (uint32_t u = 0; u < kBatch; ++u)
+  // stream's (K1024, m32 dsub 2: 8 iterations of 500,000 rows 4,850 us with all
+  // loaded at once, 4,550 one by one, of 400,000 4,140 and 3,910).
+  if constexpr (PER >= 4) {
+    for (uint32_t gg = 0; gg < G; ++gg)
 #pragma unroll
       for (uint32_t q = 0; q < PER; ++q) {
-        before[q] += g0 + u < g ? sum[u][q] : 0u;
-        tot[q] += sum[u][q];
+        const uint32_t v = q < nq ? pm[(uint64_t)gg * K + c0 + q] : 0u;
+        before[q] += gg < g ? v : 0u;
+        tot[q] += v;
+      }
+  } else {
+    uint32_t sum[kScanRanges][PER];
+#pragma unroll
+    for (uint32_t gg = 0; gg < kScanRanges; ++gg)
+#pragma unroll
+      for (uint32_t q = 0; q < PER; ++q)
+        sum[gg][q] = gg < G && q < nq ? pm[(uint64_t)gg * K + c0 + q] : 0u;
+#pragma unroll
+    for (uint32_t gg = 0; gg < kScanRanges; ++gg)
+#pragma unroll
+      for (uint32_t q = 0; q < PER; ++q) {
+        before[q] += gg < g ? sum[gg][q] : 0u;
+        tot[q] += sum[gg][q];
       }
   }
   uint32_t local = 0;
