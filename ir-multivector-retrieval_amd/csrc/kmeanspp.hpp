@@ -214,7 +214,7 @@ __device__ __forceinline__ KppDraw kpp_draw_wave(const double* __restrict__ sums
 // Bound by latency: five dependent round trips (state, run sums, the run's
 // weights, the drawn row, the rows it may lower).  As three launches (update,
 // draw, exact fallback) a round of 117,645 rows x 16 subspaces took 22 us
-// with its gaps beside the other 16's, and 13 now.
+// with its gaps beside the other 16's; this kernel takes 10.
 //
 // Without FUSED (more runs than kKppFusedRuns) kpp_draw_kernel has made the
 // draw, and no run is being read by others.
