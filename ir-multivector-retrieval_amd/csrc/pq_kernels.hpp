@@ -1304,9 +1304,9 @@ struct FoldStage {
 // Bound by latency: a prefix step per 64 chunks or binade crossing (about 18
 // crossings a fold), and by the serial adds of chunks with ties.  us a fold by
 // the event timers (which add about 5), one wave of dependent loads | this
-// with the start's binade alone | this: 117,645 chi-square terms 45 | 28 | 30;
-// 60,000,000 of them 2,490 | 28,500 | 2,130; as many equal terms 2,480 |
-// 204,000 | 2,130, and with a tie in every chunk 447,000 | 754,000 | 382,000.
+// with the start's binade alone | this: 117,645 chi-square terms 45 | 28 | 29;
+// 60,000,000 of them 2,490 | 28,500 | 2,110; as many equal terms 2,480 |
+// 204,000 | 2,080, and with a tie in every chunk 447,000 | 754,000 | 364,000.
 __device__ inline float fold_apply_block(const float* __restrict__ em, uint64_t n,
                                          const FoldChunk* __restrict__ cm,
                                          const double* __restrict__ pre, uint32_t nc,
